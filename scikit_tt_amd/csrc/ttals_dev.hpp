@@ -284,6 +284,7 @@ __device__ __forceinline__ int gmap_at(const GMap& g, int i) {
   return q * g.hi + (i - q * g.div) * g.lo;
 }
 
+typedef double dx2_t __attribute__((ext_vector_type(2)));
 typedef double dx4_t __attribute__((ext_vector_type(4)));
 typedef float fx4_t __attribute__((ext_vector_type(4)));
 
