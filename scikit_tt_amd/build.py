@@ -1,14 +1,16 @@
 """Build libttals.so in-tree for gfx950 (``python -m scikit_tt_amd.build``)."""
+import concurrent.futures
 import os
 import re
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRCS = [os.path.join(HERE, 'csrc', f) for f in ('ttals_capi.hip', 'ttals_hybrid.hip')]
+SRCS = [os.path.join(HERE, 'csrc', f) for f in ('ttals_capi.hip', 'ttals_hybrid.hip', 'ttals_tt.hip')]
 OUT = os.path.join(HERE, 'libttals.so')
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
-FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared',
+FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC',
          # MFMA results in ordinary VGPRs: accumulation registers (AGPRs) would be
          # allocated on top of the 256 VGPRs and halve the workgroups per CU
          '-mllvm', '-amdgpu-mfma-vgpr-form=1',
@@ -35,16 +37,27 @@ def build(verbose=False, out=OUT, defines=()):
     """Compile libttals.so; ``defines`` adds -D options (e.g. TTALS_PROFILE=1
     for a build whose results carry per-phase cycle counters)."""
     tmp = out + '.tmp'
-    cmd = [HIPCC] + FLAGS + ['-D' + d for d in defines] + ['-Rpass-analysis=kernel-resource-usage', '-o', tmp] + SRCS
-    if verbose:
-        print(' '.join(cmd), flush=True)
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError('hipcc failed building libttals.so')
+    opts = FLAGS + ['-D' + d for d in defines] + ['-Rpass-analysis=kernel-resource-usage']
+    with tempfile.TemporaryDirectory() as work:
+        def compile_one(src):
+            obj = os.path.join(work, os.path.basename(src) + '.o')
+            cmd = [HIPCC] + opts + ['-c', '-o', obj, src]
+            if verbose:
+                print(' '.join(cmd), flush=True)
+            return obj, subprocess.run(cmd, capture_output=True, text=True)
+
+        with concurrent.futures.ThreadPoolExecutor(len(SRCS)) as pool:
+            done = list(pool.map(compile_one, SRCS))
+        link = [HIPCC] + FLAGS + ['-shared', '-o', tmp] + [obj for obj, _ in done]
+        if all(r.returncode == 0 for _, r in done):
+            done.append((tmp, subprocess.run(link, capture_output=True, text=True)))
+    for _, r in done:
+        if r.returncode != 0:
+            sys.stderr.write(r.stdout + r.stderr)
+            raise RuntimeError('hipcc failed building libttals.so')
     os.replace(tmp, out)
     # the batched engine is sized for two resident systems per CU
-    for name, u in _resource_usage(r.stderr).items():
+    for name, u in _resource_usage(''.join(r.stderr for _, r in done)).items():
         if name.startswith('_Z5k_als') and u.get('Occupancy', 2) < 2:
             sys.stderr.write('warning: %s occupancy %d wave/SIMD (VGPRs %s, AGPRs %s): one system per CU\n'
                              % (name, u['Occupancy'], u.get('VGPRs'), u.get('AGPRs')))

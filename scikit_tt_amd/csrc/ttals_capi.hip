@@ -11,9 +11,9 @@
 #include <vector>
 
 #include "ttals_engine.hpp"
-#include "ttals_resid.hpp"
 #include "ttals_gang.hpp"
 #include "ttals_hybrid.hpp"
+#include "ttals_tt.hpp"
 #include "../../include/ttals.h"
 
 using namespace ttals;
@@ -287,246 +287,6 @@ __global__ void k_core_embed(int r0, int mn, int r1, const double* __restrict__ 
     const int q = (int)(t % mn), i = (int)(t / mn);
     dst[((long)(o0 + i) * mn + q) * R1 + (o1 + j)] = scale * src[e];
   }
-}
-
-// ||t||_2 by a right-to-left QR sweep: only the R factors are needed
-// (the norm is invariant under the orthogonal factors).  Cores are working
-// copies with dims (r, mn, r'); they are overwritten.
-struct NormArgs {
-  int d;
-  const int* mn;
-  const int* r;
-  const double* const* src;  // the caller's cores (read only)
-  double* const* c;   // working cores: c[i-1] is written when core i is absorbed
-  double* W;          // >= max_i mn_i * r_{i+1} * r_i
-  double* Rc;         // >= r_i^2
-  double* T;          // >= max_i r_{i-1} * mn_{i-1} * r_i
-  double* tau;        // >= max rank
-  double* out;
-};
-__global__ __launch_bounds__(NT) void k_tt_norm(NormArgs A) {
-  __shared__ double lds[GEMM_LDS_DOUBLES];
-  __shared__ SolveLDS S;
-  int right = A.r[A.d];
-  for (int i = A.d - 1; i >= 1; --i) {
-    const int a = A.r[i], q = A.mn[i], b = right;
-    const int m = q * b, c = a;
-    // W (m x c) = core_i^T, core_i is (a x q*b); the last core is still the caller's
-    const double* ci = (i == A.d - 1) ? A.src[i] : A.c[i];
-    for (long e = threadIdx.x; e < (long)m * c; e += NT) {
-      const int ii = (int)(e / c), jj = (int)(e % c);
-      A.W[e] = ci[(long)jj * m + ii];
-    }
-    __syncthreads();
-    wg_householder(A.W, m, c, A.tau, S.red);
-    const int k = m < c ? m : c;
-    for (long e = threadIdx.x; e < (long)k * c; e += NT) {
-      const int ii = (int)(e / c), jj = (int)(e % c);
-      A.Rc[e] = (jj >= ii) ? A.W[(long)ii * c + jj] : 0.0;
-    }
-    __syncthreads();
-    // core_{i-1} (rows x a) <- core_{i-1} * R^T  (rows x k)
-    const int rows = A.r[i - 1] * A.mn[i - 1];
-    wg_gemm<double, double>(rows, k, a, crm<double>(A.src[i - 1], a), ctr<double>(A.Rc, c), mrm<double>(A.T, k),
-                            lds);
-    wg_copy(A.T, A.c[i - 1], rows * k);
-    __syncthreads();
-    right = k;
-  }
-  const long n0 = (long)A.r[0] * A.mn[0] * right;
-  const double nrm = wg_nrm2(A.d == 1 ? A.src[0] : A.c[0], (int)n0, S.red);
-  if (threadIdx.x == 0) A.out[0] = nrm;
-}
-
-// Left/right orthonormalisation sweep of a TT (one workgroup).  Cores are
-// updated in place (capacity of the input ranks); ranks (device int[d+1]) are
-// updated.  dims: mn[i] = m_i * n_i.
-//   no truncation: Householder QR of the tall unfolding, Q kept, R pushed on;
-//   truncation (threshold > 0 or a finite max rank): the same QR, then a
-//   one-sided Jacobi SVD of R, singular triplets with s/s0 > threshold (then
-//   at most max_rank[bond]) kept, S V^T (or U S) pushed on
-//   (scikit_tt/tensor_train.py:1162-1189, 1268-1299).
-struct OrthoArgs {
-  int d, dir, start, end;  // dir 0: left (i = start..end), 1: right (i = start..end descending)
-  int trunc;
-  double thr;
-  const int* maxr;  // [d+1], <= 0 = unbounded
-  const int* mn;
-  int* r;
-  double* const* c;
-  double* W;   // >= max core size
-  double* Qm;  // >= max core size
-  double* Rc;  // >= rmax^2
-  double* T;   // >= max core size
-  double* tau; // >= rmax
-  double* Bm;  // >= rmax^2
-  double* Vm;  // >= rmax^2
-  double* sig; // >= rmax
-  int* perm;   // >= rmax
-};
-
-// T (mt x ct) tall unfolding in A.W; on return the kept left factor
-// (mt x kk, row-major) is in A.Qm and the pushed factor in A.Bm:
-// B[:, perm] (ct x kk, row-major, ld kk).  Returns kk.
-__device__ int ortho_factor(const OrthoArgs& A, int mt, int ct, int cap, double* lds, SolveLDS& S) {
-  wg_householder(A.W, mt, ct, A.tau, S.red);
-  wg_form_q(A.W, mt, ct, A.tau, A.T);  // Q (mt x k) in T
-  const int k = mt < ct ? mt : ct;
-  if (!A.trunc) {
-    for (long e = threadIdx.x; e < (long)k * ct; e += NT) {
-      const int ii = (int)(e / ct), jj = (int)(e % ct);
-      A.Rc[e] = (jj >= ii) ? A.W[(long)ii * ct + jj] : 0.0;
-    }
-    wg_copy(A.T, A.Qm, mt * k);
-    // pushed factor R^T (ct x k)
-    for (long e = threadIdx.x; e < (long)ct * k; e += NT) {
-      const int ii = (int)(e / k), jj = (int)(e % k);
-      A.Bm[e] = A.Rc[(long)jj * ct + ii];
-    }
-    __syncthreads();
-    return k;
-  }
-  // B = R^T (ct x k); Jacobi: B = U_B S, V
-  for (long e = threadIdx.x; e < (long)ct * k; e += NT) {
-    const int ii = (int)(e / k), jj = (int)(e % k);
-    A.Rc[e] = (ii >= jj) ? A.W[(long)jj * ct + ii] : 0.0;
-  }
-  __syncthreads();
-  wg_jacobi_svd(A.Rc, ct, k, A.Vm, A.sig, A.perm, S.red);
-  // number kept: s/s0 > thr, then the cap
-  int kk = 0;
-  const double s0 = A.sig[A.perm[0]];
-  for (int j = 0; j < k; ++j)
-    if (A.thr == 0.0 || A.sig[A.perm[j]] / s0 > A.thr) ++kk;
-  if (cap > 0 && kk > cap) kk = cap;
-  if (kk < 1) kk = 1;
-  // left factor (Q V)[:, perm[:kk]] -> Qm (mt x kk)
-  wg_gemm<double, double>(mt, k, k, crm<double>(A.T, k), crm<double>(A.Vm, k), mrm<double>(A.W, k), lds);
-  for (long e = threadIdx.x; e < (long)mt * kk; e += NT) {
-    const int ii = (int)(e / kk), jj = (int)(e % kk);
-    A.Qm[e] = A.W[(long)ii * k + A.perm[jj]];
-  }
-  // pushed factor B[:, perm[:kk]] (ct x kk)
-  for (long e = threadIdx.x; e < (long)ct * kk; e += NT) {
-    const int ii = (int)(e / kk), jj = (int)(e % kk);
-    A.Bm[e] = A.Rc[(long)ii * k + A.perm[jj]];
-  }
-  __syncthreads();
-  return kk;
-}
-
-__global__ __launch_bounds__(NT) void k_tt_ortho(OrthoArgs A) {
-  __shared__ double lds[GEMM_LDS_DOUBLES];
-  __shared__ SolveLDS S;
-  if (A.dir == 0) {
-    for (int i = A.start; i <= A.end; ++i) {
-      const int a = A.r[i], q = A.mn[i], b = A.r[i + 1];
-      const int m = a * q, c = b;
-      wg_copy(A.c[i], A.W, m * c);
-      __syncthreads();
-      const int k = ortho_factor(A, m, c, A.maxr[i + 1], lds, S);
-      wg_copy(A.Qm, A.c[i], m * k);
-      __syncthreads();
-      // core_{i+1} (b x rest) <- Bm^T (k x b) * core_{i+1}
-      const int rest = A.mn[i + 1] * A.r[i + 2];
-      wg_gemm<double, double>(k, rest, b, ctr<double>(A.Bm, k), crm<double>(A.c[i + 1], rest),
-                              mrm<double>(A.T, rest), lds);
-      wg_copy(A.T, A.c[i + 1], k * rest);
-      if (threadIdx.x == 0) A.r[i + 1] = k;
-      __syncthreads();
-    }
-  } else {
-    for (int i = A.start; i >= A.end; --i) {
-      const int a = A.r[i], q = A.mn[i], b = A.r[i + 1];
-      const int m = q * b, c = a;
-      for (long e = threadIdx.x; e < (long)m * c; e += NT) {
-        const int ii = (int)(e / c), jj = (int)(e % c);
-        A.W[e] = A.c[i][(long)jj * m + ii];
-      }
-      __syncthreads();
-      const int k = ortho_factor(A, m, c, A.maxr[i], lds, S);
-      // core_i (k x m) = Qm^T
-      for (long e = threadIdx.x; e < (long)k * m; e += NT) {
-        const int rr = (int)(e / m), cc = (int)(e % m);
-        A.c[i][e] = A.Qm[(long)cc * k + rr];
-      }
-      __syncthreads();
-      const int rows = A.r[i - 1] * A.mn[i - 1];
-      wg_gemm<double, double>(rows, k, a, crm<double>(A.c[i - 1], a), crm<double>(A.Bm, k), mrm<double>(A.T, k),
-                              lds);
-      wg_copy(A.T, A.c[i - 1], rows * k);
-      if (threadIdx.x == 0) A.r[i] = k;
-      __syncthreads();
-    }
-  }
-}
-
-// Truncated SVD of a row-major m x c matrix Y (one workgroup): Householder
-// QR of the tall orientation (Y, or Y^T when m < c), one-sided Jacobi SVD of
-// R^T, singular triplets kept by s/s0 > thr (rel) or s > thr (absolute) when
-// thr != 0, then at most maxr (the rule of scikit_tt/utils.py:145-156).
-// U (m x k), s (k), Vt (k x c) row-major; k written to *kout.
-struct SvdArgs {
-  int m, c, maxr, rel;
-  double thr;
-  const double* Y;
-  double* U;
-  double* s;
-  double* Vt;
-  double* W;    // mt x ct
-  double* Qm;   // mt x ct
-  double* B;    // ct x ct
-  double* Vm;   // ct x ct
-  double* L;    // mt x ct
-  double* sig;  // ct
-  double* tau;  // ct
-  int* perm;    // ct
-  int* kout;
-};
-__global__ __launch_bounds__(NT) void k_svd_trunc(SvdArgs A) {
-  __shared__ double lds[GEMM_LDS_DOUBLES];
-  __shared__ double red[4 * NWAVE];
-  const bool tall = A.m >= A.c;
-  const int mt = tall ? A.m : A.c, ct = tall ? A.c : A.m;
-  for (long e = threadIdx.x; e < (long)mt * ct; e += NT) {
-    const int i = (int)(e / ct), j = (int)(e % ct);
-    A.W[e] = tall ? A.Y[e] : A.Y[(long)j * A.c + i];
-  }
-  __syncthreads();
-  wg_householder(A.W, mt, ct, A.tau, red);
-  wg_form_q(A.W, mt, ct, A.tau, A.Qm);
-  // B = R^T (ct x ct)
-  for (long e = threadIdx.x; e < (long)ct * ct; e += NT) {
-    const int i = (int)(e / ct), j = (int)(e % ct);
-    A.B[e] = (i >= j) ? A.W[(long)j * ct + i] : 0.0;
-  }
-  __syncthreads();
-  wg_jacobi_svd(A.B, ct, ct, A.Vm, A.sig, A.perm, red);
-  int kk = 0;
-  const double s0 = A.sig[A.perm[0]];
-  for (int j = 0; j < ct; ++j) {
-    const double sj = A.sig[A.perm[j]];
-    if (A.thr == 0.0 || (A.rel ? (s0 > 0.0 && sj / s0 > A.thr) : sj > A.thr)) ++kk;
-  }
-  if (A.maxr > 0 && kk > A.maxr) kk = A.maxr;
-  // left factor of the tall orientation: (Q V)[:, perm[:kk]] (mt x kk)
-  wg_gemm<double, double>(mt, ct, ct, crm<double>(A.Qm, ct), crm<double>(A.Vm, ct), mrm<double>(A.L, ct), lds);
-  for (long e = threadIdx.x; e < (long)mt * kk; e += NT) {
-    const int i = (int)(e / kk), j = (int)(e % kk);
-    const double v = A.L[(long)i * ct + A.perm[j]];
-    if (tall) A.U[(long)i * kk + j] = v;       // U = left factor
-    else A.Vt[(long)j * mt + i] = v;            // Vt = (left factor)^T
-  }
-  // right factor: B[:, perm[j]] / s (ct x kk)
-  for (long e = threadIdx.x; e < (long)ct * kk; e += NT) {
-    const int i = (int)(e / kk), j = (int)(e % kk);
-    const double sj = A.sig[A.perm[j]];
-    const double v = sj > 0.0 ? A.B[(long)i * ct + A.perm[j]] / sj : 0.0;
-    if (tall) A.Vt[(long)j * ct + i] = v;       // Vt = (right factor)^T
-    else A.U[(long)i * kk + j] = v;             // U = right factor
-  }
-  for (int j = threadIdx.x; j < kk; j += NT) A.s[j] = A.sig[A.perm[j]];
-  if (threadIdx.x == 0) *A.kout = kk;
 }
 
 // Householder reduction of C (N x N, row-major, global memory) to upper
@@ -2635,8 +2395,7 @@ int ttals_tt_norm(ttals_ctx* c, void* stream, const ttals_tt* t, double* out) {
   na.T = reinterpret_cast<double*>(db + oT);
   na.tau = reinterpret_cast<double*>(db + otau);
   na.out = reinterpret_cast<double*>(db + oout);
-  hipLaunchKernelGGL(k_tt_norm, dim3(1), dim3(NT), 0, st, na);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, tt_norm_launch(st, na));
   double h = 0.0;
   HIPCHK(c, hipMemcpyAsync(&h, na.out, 8, hipMemcpyDeviceToHost, st));
   HIPCHK(c, hipStreamSynchronize(st));
@@ -2735,8 +2494,7 @@ int ttals_residual_norm_batch(ttals_ctx* c, void* stream, int count, const ttals
     D.out = dres + 2 * s;
   }
   HIPCHK(c, hipMemcpyAsync(dmeta, c->hst, meta_bytes, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_residual_norm, dim3(count), dim3(NT), 0, st, (const ResidDesc*)dmeta);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, residual_norm_launch(count, st, (const ResidDesc*)dmeta));
   HIPCHK(c, hipMemcpyAsync(c->hst + r_out, dres, 8 * 2 * (size_t)count, hipMemcpyDeviceToHost, st));
   HIPCHK(c, hipStreamSynchronize(st));
   const double* h = hptr<double>(c, r_out);
@@ -2758,7 +2516,7 @@ int ttals_truncated_svd(ttals_ctx* c, void* stream, int m, int cdim, const doubl
   Layout L;
   const size_t oW = L.take(8 * mt * ct), oQ = L.take(8 * mt * ct), oB = L.take(8 * ct * ct), oV = L.take(8 * ct * ct),
                oL = L.take(8 * mt * ct), osig = L.take(8 * ct), otau = L.take(8 * ct), operm = L.take(4 * ct),
-               ok = L.take(8);
+               ok = L.take(8), oTg = L.take(8 * qr_tg_doubles(ct));
   int rc;
   if ((rc = ensure_dws(c, L.bytes))) return rc;
   char* db = reinterpret_cast<char*>(c->dws);
@@ -2781,9 +2539,9 @@ int ttals_truncated_svd(ttals_ctx* c, void* stream, int m, int cdim, const doubl
   a.tau = reinterpret_cast<double*>(db + otau);
   a.perm = reinterpret_cast<int*>(db + operm);
   a.kout = reinterpret_cast<int*>(db + ok);
+  a.Tg = reinterpret_cast<double*>(db + oTg);
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(k_svd_trunc, dim3(1), dim3(NT), 0, st, a);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, svd_trunc_launch(st, a));
   int h = 0;
   HIPCHK(c, hipMemcpyAsync(&h, a.kout, sizeof(int), hipMemcpyDeviceToHost, st));
   HIPCHK(c, hipStreamSynchronize(st));
@@ -2888,7 +2646,7 @@ int ttals_tt_ortho(ttals_ctx* c, void* stream, const ttals_tt* t, int dir, int s
   Layout L;
   const size_t oW = L.take(8 * cmax), oQ = L.take(8 * cmax), oR = L.take(8 * rmax * rmax), oT = L.take(8 * cmax),
                otau = L.take(8 * rmax), oB = L.take(8 * rmax * rmax), oV = L.take(8 * rmax * rmax),
-               osig = L.take(8 * rmax), operm = L.take(sizeof(int) * rmax);
+               osig = L.take(8 * rmax), operm = L.take(sizeof(int) * rmax), oTg = L.take(8 * qr_tg_doubles(rmax));
   const size_t omn = L.take(sizeof(int) * d), orr = L.take(sizeof(int) * (d + 1)), omx = L.take(sizeof(int) * (d + 1)),
                optr = L.take(sizeof(void*) * d);
   if ((rc = ensure_dws(c, L.bytes))) return rc;
@@ -2927,8 +2685,8 @@ int ttals_tt_ortho(ttals_ctx* c, void* stream, const ttals_tt* t, int dir, int s
   oa.Vm = reinterpret_cast<double*>(db + oV);
   oa.sig = reinterpret_cast<double*>(db + osig);
   oa.perm = reinterpret_cast<int*>(db + operm);
-  hipLaunchKernelGGL(k_tt_ortho, dim3(1), dim3(NT), 0, st, oa);
-  HIPCHK(c, hipGetLastError());
+  oa.Tg = reinterpret_cast<double*>(db + oTg);
+  HIPCHK(c, tt_ortho_launch(st, oa));
   HIPCHK(c, hipMemcpyAsync(c->hst + orr, db + orr, sizeof(int) * (d + 1), hipMemcpyDeviceToHost, st));
   HIPCHK(c, hipStreamSynchronize(st));
   for (int i = 0; i <= d; ++i) t->ranks[i] = hrr[i];

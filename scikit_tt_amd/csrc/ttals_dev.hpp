@@ -12,8 +12,14 @@
 
 namespace ttals {
 
-constexpr int NT = 256;            // threads per workgroup: 4 x wave64
+// Threads per workgroup: 4 waves, or 8 in a translation unit that defines
+// TTALS_NT 512 for kernels whose workgroup has a CU to itself.
+#ifndef TTALS_NT
+#define TTALS_NT 256
+#endif
+constexpr int NT = TTALS_NT;
 constexpr int NWAVE = NT / 64;
+static_assert(NT == 256 || NT == 512, "the tile shapes below assume 4 or 8 waves");
 
 // ---------------------------------------------------------------------------
 // index maps: a matrix row (or column) index i is split into
@@ -260,11 +266,11 @@ __device__ __forceinline__ void wg_fill(T* y, T v, int n) {
 }
 
 // ---------------------------------------------------------------------------
-// Workgroup GEMM  C[M x N] = A[M x K] * B[K x N]  (T = storage/compute type,
-// accumulation in ACC).  64x64 output tiles, K-steps of 16 staged in LDS;
-// each thread owns a 4x4 register micro-tile.
+// Workgroup GEMM  C[M x N] = A[M x K] * B[K x N].  GBM x GBN output tiles
+// (64 x 64 with four waves, 128 x 64 with eight), K-steps of 16 staged in LDS,
+// a 32 x 32 quadrant per wave.
 
-constexpr int GBM = 64, GBN = 64, GBK = 16;
+constexpr int GBM = NT / 4, GBN = 64, GBK = 16;
 constexpr int GEMM_LDS_DOUBLES = GBK * (GBM + 1) + GBK * (GBN + 1);
 
 // i -> (i / div) * hi + (i % div) * lo for 0 <= i < 2^22 with an FP32
@@ -313,7 +319,7 @@ __device__ __forceinline__ int mfma16_row(int lk, int e) {
 #endif
 constexpr int GEMM_PREFETCH = TTALS_GEMM_PREFETCH;
 
-// FP64 GEMM over global (L2/HBM) operands on the matrix cores.  64x64 output
+// FP64 GEMM over global (L2/HBM) operands on the matrix cores.  GBM x 64 output
 // tiles, K-steps of 16 staged through LDS ([GBK][GBM+1] and [GBK][GBN+1]:
 // the odd stride keeps the transposing stores of k-fast operands off a single
 // bank); every wave owns a 32x32 quadrant of the tile (2x2
@@ -328,19 +334,21 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
   typedef typename std::conditional<std::is_same<T, double>::value, dx4_t, fx4_t>::type acc_t;
   TT_LDS T* As = (TT_LDS T*)lds_;              // [GBK][GBM+1]
   TT_LDS T* Bs = (TT_LDS T*)lds_ + GBK * (GBM + 1);  // [GBK][GBN+1]
-  static_assert(GBM == 64 && GBN == 64 && GBK == 16 && NT == 256, "tile shape assumed below");
+  static_assert(GBM == NT / 4 && GBN == 64 && GBK == 16, "tile shape assumed below");
+  constexpr int WM = GBM / 32;                 // waves along M
+  constexpr int NB_LD = GBN * GBK / NT;        // B elements a thread loads per K-step (A: 4)
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, lk = lane >> 4;
-  const int wm = (w & 1) << 5, wn = (w >> 1) << 5;
+  const int wm = (w % WM) << 5, wn = (w / WM) << 5;
   const GMap Ar = gmap(A.r), Ac = gmap(A.c), Br = gmap(B.r), Bc = gmap(B.c);
   // contiguous direction of each operand decides which index is thread-fast (coalescing)
   const bool a_kfast = (A.c.lo == 1 && A.c.div >= K);
   const bool b_nfast = (B.c.lo == 1 && B.c.div >= N);
-  // per-thread element coordinates in a (64 x 16) / (16 x 64) stage, j = 0..3
-  const int a_i0 = a_kfast ? (tid >> 4) : (tid & 63), a_k0 = a_kfast ? (tid & 15) : (tid >> 6);
-  const int a_di = a_kfast ? 16 : 0, a_dk = a_kfast ? 0 : 4;
+  // per-thread element coordinates in a (GBM x 16) / (16 x 64) stage
+  const int a_i0 = a_kfast ? (tid >> 4) : (tid & (GBM - 1)), a_k0 = a_kfast ? (tid & 15) : tid / GBM;
+  const int a_di = a_kfast ? NT / 16 : 0, a_dk = a_kfast ? 0 : NT / GBM;
   const int b_n0 = b_nfast ? (tid & 63) : (tid >> 4), b_k0 = b_nfast ? (tid >> 6) : (tid & 15);
-  const int b_dn = b_nfast ? 0 : 16, b_dk = b_nfast ? 4 : 0;
+  const int b_dn = b_nfast ? 0 : NT / 16, b_dk = b_nfast ? NT / 64 : 0;
   const int tn = (N + GBN - 1) / GBN, ks = (K + GBK - 1) / GBK;
   const int steps = ((M + GBM - 1) / GBM) * tn * ks;
   // loader position (tile origin, K offset) and compute position, advanced without division
@@ -350,12 +358,13 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
   // arithmetic (a wave-uniform branch)
   const bool a_plain = A.r.div >= (1 << 22) && A.c.div >= (1 << 22);
   const bool b_plain = B.r.div >= (1 << 22) && B.c.div >= (1 << 22);
-  auto load = [&](T (&ra)[4], T (&rb)[4]) {
+  auto load = [&](T (&ra)[4], T (&rb)[NB_LD]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int gm = lm0 + a_i0 + j * a_di, gk = lk0 + a_k0 + j * a_dk;
       const int ao = a_plain ? gm * A.r.lo + gk * A.c.lo : gmap_at(Ar, gm) + gmap_at(Ac, gk);
       ra[j] = (gm < M && gk < K) ? A.p[ao] : (T)0;
+      if (j >= NB_LD) continue;
       const int gn = ln0 + b_n0 + j * b_dn, gk2 = lk0 + b_k0 + j * b_dk;
       const int bo = b_plain ? gk2 * B.r.lo + gn * B.c.lo : gmap_at(Br, gk2) + gmap_at(Bc, gn);
       rb[j] = (gn < N && gk2 < K) ? B.p[bo] : (T)0;
@@ -371,11 +380,11 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
       }
     }
   };
-  auto stage = [&](const T (&ra)[4], const T (&rb)[4]) {
+  auto stage = [&](const T (&ra)[4], const T (&rb)[NB_LD]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       As[(a_k0 + j * a_dk) * (GBM + 1) + a_i0 + j * a_di] = ra[j];
-      Bs[(b_k0 + j * b_dk) * (GBN + 1) + b_n0 + j * b_dn] = rb[j];
+      if (j < NB_LD) Bs[(b_k0 + j * b_dk) * (GBN + 1) + b_n0 + j * b_dn] = rb[j];
     }
   };
   acc_t acc[2][2];
@@ -425,7 +434,7 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
   };
   if constexpr (GEMM_PREFETCH == 2) {
     // two register sets: while step s computes, steps s+1 and s+2 are loading
-    T ra0[4], rb0[4], ra1[4], rb1[4];
+    T ra0[4], rb0[NB_LD], ra1[4], rb1[NB_LD];
     if (steps > 0) {
       load(ra0, rb0);
       stage(ra0, rb0);
@@ -448,7 +457,7 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
       }
     }
   } else {
-    T ra[4], rb[4];
+    T ra[4], rb[NB_LD];
     if (steps > 0) {
       load(ra, rb);
       stage(ra, rb);
@@ -501,79 +510,21 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
   }
 }
 
-template <class T, class ACC>
-__device__ void wg_gemm_valu(int M, int N, int K, CView<T> A, CView<T> B, MView<T> C, ACC* lds);
-
-// GEMM over global operands: the matrix cores in FP64 or FP32 (accumulating
-// in the operands' precision), the vector units (register tiles) otherwise.
+// GEMM over global operands on the matrix cores, FP64 or FP32 (accumulating
+// in the operands' precision).
 template <class T, class ACC>
 __device__ void wg_gemm(int M, int N, int K, CView<T> A, CView<T> B, MView<T> C, ACC* lds) {
-  if constexpr ((std::is_same<T, double>::value || std::is_same<T, float>::value) && std::is_same<ACC, T>::value)
+  static_assert((std::is_same<T, double>::value || std::is_same<T, float>::value) && std::is_same<ACC, T>::value,
+                "matrix-core GEMM in the operands' precision");
+  if constexpr (GBM > GBN) {
+    // the longer output side along the tile's longer side: C^T = B^T A^T
+    const bool sw = M <= GBN && N > M;
+    const CView<T> At{A.p, A.c, A.r}, Bt{B.p, B.c, B.r};
+    wg_gemm_mf<T>(sw ? N : M, sw ? M : N, K, sw ? Bt : A, sw ? At : B, MView<T>{C.p, sw ? C.c : C.r, sw ? C.r : C.c},
+                  lds);
+  } else {
     wg_gemm_mf<T>(M, N, K, A, B, C, lds);
-  else
-    wg_gemm_valu<T, ACC>(M, N, K, A, B, C, lds);
-}
-
-template <class T, class ACC>
-__device__ void wg_gemm_valu(int M, int N, int K, CView<T> A, CView<T> B, MView<T> C, ACC* lds) {
-  ACC* As = lds;                      // [GBK][GBM+1]
-  ACC* Bs = lds + GBK * (GBM + 1);    // [GBK][GBN+1]
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;
-  const GMap Ar = gmap(A.r), Ac = gmap(A.c), Br = gmap(B.r), Bc = gmap(B.c);
-  // contiguous direction of each operand decides the load order (coalescing)
-  const bool a_kfast = (A.c.lo == 1 && A.c.div >= K);
-  const bool b_nfast = (B.c.lo == 1 && B.c.div >= N);
-  for (int m0 = 0; m0 < M; m0 += GBM) {
-    for (int n0 = 0; n0 < N; n0 += GBN) {
-      ACC acc[4][4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] = (ACC)0;
-      for (int k0 = 0; k0 < K; k0 += GBK) {
-        for (int e = tid; e < GBM * GBK; e += NT) {
-          int mi, ki;
-          if (a_kfast) { ki = e % GBK; mi = e / GBK; } else { mi = e % GBM; ki = e / GBM; }
-          const int gm = m0 + mi, gk = k0 + ki;
-          As[ki * (GBM + 1) + mi] = (gm < M && gk < K) ? (ACC)A.p[gmap_at(Ar, gm) + gmap_at(Ac, gk)] : (ACC)0;
-        }
-        for (int e = tid; e < GBN * GBK; e += NT) {
-          int ni, ki;
-          if (b_nfast) { ni = e % GBN; ki = e / GBN; } else { ki = e % GBK; ni = e / GBK; }
-          const int gn = n0 + ni, gk = k0 + ki;
-          Bs[ki * (GBN + 1) + ni] = (gn < N && gk < K) ? (ACC)B.p[gmap_at(Br, gk) + gmap_at(Bc, gn)] : (ACC)0;
-        }
-        __syncthreads();
-        const int kmax = (K - k0) < GBK ? (K - k0) : GBK;
-        for (int kk = 0; kk < kmax; ++kk) {
-          ACC a[4], b[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) a[r] = As[kk * (GBM + 1) + ty + 16 * r];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) b[c] = Bs[kk * (GBN + 1) + tx + 16 * c];
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[r][c] += a[r] * b[c];
-        }
-        __syncthreads();
-      }
-      const GMap Cr = gmap(C.r), Cc = gmap(C.c);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gm = m0 + ty + 16 * r;
-        if (gm >= M) continue;
-        const int cr = gmap_at(Cr, gm);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int gn = n0 + tx + 16 * c;
-          if (gn < N) C.p[cr + gmap_at(Cc, gn)] = (T)acc[r][c];
-        }
-      }
-    }
   }
-  __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -792,13 +743,15 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
   // no integer divisions below (each expands to a long instruction sequence):
   // tile rows by an FP32-reciprocal quotient (exact for these small counts),
   // the K-split cases by shifts
-  static_assert(NWAVE == 4, "the K-split cases assume four waves");
   const int tn = (N + 15) >> 4, tiles = ((M + 15) >> 4) * tn;
   const float itn = 1.0f / (float)tn;
   const int ks = (K + 3) >> 2;
-  int gl = 0;  // log2 of the K groups: tiles == 1 -> 4 groups, tiles == 2 -> 2 (every wave one (tile, part))
-  if (tiles <= 2) {
-    gl = tiles == 1 ? 2 : 1;
+  // log2 of the K groups: 1, 2 (and with eight waves 4) tiles split their K
+  // range so that every wave has one (tile, part)
+  const int tl = tiles == 1 ? 0 : (tiles == 2 ? 1 : 2);  // log2 of a splitting tile count
+  int gl = 0;
+  if (2 * tiles <= NWAVE && (tiles & (tiles - 1)) == 0) {
+    gl = (NWAVE == 8 ? 3 : 2) - tl;
     if (((1 << gl) - 1) * tiles * 256 > red_cap) gl = 0;
   }
   const int groups = 1 << gl;
@@ -882,9 +835,9 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
     return;
   }
   for (int u = w; u < tiles * groups; u += NWAVE) {
-    // groups > 1 only with tiles 1 or 2
-    const int t = gl == 0 ? u : (tiles == 1 ? 0 : (u & 1));
-    const int part = gl == 0 ? 0 : (tiles == 1 ? u : (u >> 1));
+    // groups > 1 only with a power of two of tiles
+    const int t = gl == 0 ? u : (u & (tiles - 1));
+    const int part = gl == 0 ? 0 : (u >> tl);
     const int ti = (int)(((float)t + 0.5f) * itn), tj = t - ti * tn;
     const int i = (ti << 4) + li, j = (tj << 4) + li;
     const bool iv = i < M, jv = j < N;

@@ -48,3 +48,49 @@ def test_core_product(lib, n, r1, m, r2, s1, p, s2, shift):
     torch.cuda.synchronize()
     bound = n * EPS * product(A.abs(), X.abs())
     assert bool(((out - product(A, X)).abs() <= bound).all())
+
+
+# (m, c) of one panel: edges of the 16-column blocks, of the 16-row blocks, of the
+# register forms (256, 512, 1024, 1536 rows) and of the rows one call holds (2304)
+PANELS = [(1, 1), (5, 3), (16, 16), (17, 16), (16, 17), (20, 40), (33, 31), (255, 17), (257, 33), (512, 64), (513, 65),
+          (1025, 20), (1537, 7), (2304, 18), (2305, 18), (5000, 40)]
+
+
+@pytest.mark.parametrize('m,c', PANELS)
+def test_panel_qr(lib, m, c):
+    """Householder QR of one panel: the second core of a two-core train is the
+    panel's transpose.  Norm (R only) and, where Q is formed, ortho_right:
+    orthonormal rows and the same tensor, to c * m eps (Householder QR is
+    backward stable: a modest multiple of it is the error bound)."""
+    from scikit_tt_amd.tensor_train import TT
+    gen = torch.Generator(device='cuda').manual_seed(m * 1000 + c)
+    a, b = _randn(gen, 1, 3, 1, c), _randn(gen, c, m, 1, 1)
+    full = a.view(3, c) @ b.view(c, m)
+    tol = 4 * m * c * EPS
+    assert abs(TT([a, b]).norm() - float(full.norm())) <= tol * float(full.norm())
+    t = TT([a.clone(), b.clone()]).ortho_right()
+    q = t.device_cores[1].reshape(t.ranks[1], m)
+    assert t.ranks == [1, min(m, c), 1]
+    assert float((q @ q.T - torch.eye(min(m, c), dtype=torch.float64, device='cuda')).abs().max()) <= tol
+    assert float((t.device_cores[0].view(3, -1) @ q - full).norm()) <= tol * float(full.norm())
+    # the reflectors' sign convention: R's first diagonal entry is -sign(pivot) |column|, or the pivot itself where
+    # nothing lies below it (a one-row panel)
+    ref = b.view(c, m)[0]
+    first = -torch.sign(ref[0]) * ref / ref.norm() if m > 1 else torch.ones_like(ref)
+    assert float((q[0] - first).norm()) <= tol
+
+
+def test_panel_qr_of_zero_and_repeated_columns(lib):
+    """Exactly reduced columns (H_j = I) and rank-deficient panels keep Q orthonormal and the tensor."""
+    from scikit_tt_amd.tensor_train import TT
+    gen = torch.Generator(device='cuda').manual_seed(1)
+    b = _randn(gen, 24, 300, 1, 1)
+    b[5] = 0.0
+    b[17:] = b[:7]
+    a = _randn(gen, 1, 2, 1, 24)
+    full = a.view(2, 24) @ b.view(24, 300)
+    t = TT([a.clone(), b.clone()]).ortho_right()
+    q = t.device_cores[1].reshape(24, 300)
+    tol = 4 * 24 * 300 * EPS
+    assert float((q @ q.T - torch.eye(24, dtype=torch.float64, device='cuda')).abs().max()) <= tol
+    assert float((t.device_cores[0].view(2, 24) @ q - full).norm()) <= tol * float(full.norm())
