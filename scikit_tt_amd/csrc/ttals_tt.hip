@@ -10,6 +10,7 @@
 
 #include "ttals_dev.hpp"
 #include "ttals_qr.hpp"
+#include "ttals_svd.hpp"
 
 namespace ttals {
 
@@ -19,6 +20,26 @@ struct TtLDS {
   double* gemm;
 };
 constexpr size_t TT_LDS_BYTES = sizeof(HqLDS) > 8 * GEMM_LDS_DOUBLES ? sizeof(HqLDS) : 8 * GEMM_LDS_DOUBLES;
+// kernels with an SVD: factors of up to 96 x 96 in LDS (one workgroup per CU either way)
+constexpr size_t SVD_LDS_BYTES = 152 * 1024;
+static_assert(SVD_LDS_BYTES >= TT_LDS_BYTES, "the QR's block and the GEMM tiles fit too");
+
+// SVD of the factor B (c x k, row-major) as B V = U diag(sig): in LDS where B
+// and V fit it, else in global memory, a wave per column pair.
+__device__ void jacobi_svd(double* B, int c, int k, double* V, double* sig, int* perm, const TtLDS& S, double* red) {
+  if (js_fits(c, k, SVD_LDS_BYTES / 8)) wg_jacobi_lds(B, c, k, V, sig, perm, S.gemm);
+  else wg_jacobi_svd(B, c, k, V, sig, perm, red);
+}
+
+// How many of the k singular values (sorted by perm) pass: s/s0 > thr (rel) or
+// s > thr, all of them when thr is 0.
+__device__ int count_kept(const double* sig, const int* perm, int k, double thr, bool rel, double* red) {
+  const double s0 = sig[perm[0]];
+  double n = 0.0;
+  for (int j = threadIdx.x; j < k; j += NT)
+    if (thr == 0.0 || (rel ? sig[j] / s0 > thr : sig[j] > thr)) n += 1.0;
+  return (int)wg_sum(n, red);
+}
 
 // R of the QR of the panel W (m x c, row-major, overwritten): in the top rows
 // of the returned matrix (row stride c).  Panels of more columns than half
@@ -183,12 +204,9 @@ __device__ int ortho_factor(const OrthoArgs& A, int mt, int ct, int cap, const T
     A.Rc[e] = (ii >= jj) ? A.W[(long)jj * ct + ii] : 0.0;
   }
   __syncthreads();
-  wg_jacobi_svd(A.Rc, ct, k, A.Vm, A.sig, A.perm, red);
+  jacobi_svd(A.Rc, ct, k, A.Vm, A.sig, A.perm, S, red);
   // number kept: s/s0 > thr, then the cap
-  int kk = 0;
-  const double s0 = A.sig[A.perm[0]];
-  for (int j = 0; j < k; ++j)
-    if (A.thr == 0.0 || A.sig[A.perm[j]] / s0 > A.thr) ++kk;
+  int kk = count_kept(A.sig, A.perm, k, A.thr, true, red);
   if (cap > 0 && kk > cap) kk = cap;
   if (kk < 1) kk = 1;
   // left factor (Q V)[:, perm[:kk]] -> Qm (mt x kk)
@@ -271,13 +289,8 @@ __global__ __launch_bounds__(NT) void k_svd_trunc(SvdArgs A) {
     A.B[e] = (i >= j) ? A.W[(long)j * ct + i] : 0.0;
   }
   __syncthreads();
-  wg_jacobi_svd(A.B, ct, ct, A.Vm, A.sig, A.perm, red);
-  int kk = 0;
-  const double s0 = A.sig[A.perm[0]];
-  for (int j = 0; j < ct; ++j) {
-    const double sj = A.sig[A.perm[j]];
-    if (A.thr == 0.0 || (A.rel ? (s0 > 0.0 && sj / s0 > A.thr) : sj > A.thr)) ++kk;
-  }
+  jacobi_svd(A.B, ct, ct, A.Vm, A.sig, A.perm, S, red);
+  int kk = count_kept(A.sig, A.perm, ct, A.thr, A.rel != 0, red);
   if (A.maxr > 0 && kk > A.maxr) kk = A.maxr;
   // left factor of the tall orientation: (Q V)[:, perm[:kk]] (mt x kk)
   wg_gemm<double, double>(mt, ct, ct, crm<double>(A.Qm, ct), crm<double>(A.Vm, ct), mrm<double>(A.L, ct), S.gemm);
@@ -308,11 +321,11 @@ hipError_t tt_norm_launch(hipStream_t stream, const NormArgs& a) {
   return hipGetLastError();
 }
 hipError_t tt_ortho_launch(hipStream_t stream, const OrthoArgs& a) {
-  hipLaunchKernelGGL(k_tt_ortho, dim3(1), dim3(NT), TT_LDS_BYTES, stream, a);
+  hipLaunchKernelGGL(k_tt_ortho, dim3(1), dim3(NT), SVD_LDS_BYTES, stream, a);
   return hipGetLastError();
 }
 hipError_t svd_trunc_launch(hipStream_t stream, const SvdArgs& a) {
-  hipLaunchKernelGGL(k_svd_trunc, dim3(1), dim3(NT), TT_LDS_BYTES, stream, a);
+  hipLaunchKernelGGL(k_svd_trunc, dim3(1), dim3(NT), SVD_LDS_BYTES, stream, a);
   return hipGetLastError();
 }
 

@@ -94,3 +94,35 @@ def test_panel_qr_of_zero_and_repeated_columns(lib):
     tol = 4 * 24 * 300 * EPS
     assert float((q @ q.T - torch.eye(24, dtype=torch.float64, device='cuda')).abs().max()) <= tol
     assert float((t.device_cores[0].view(2, 24) @ q - full).norm()) <= tol * float(full.norm())
+
+
+@pytest.mark.parametrize('m,c', [(1, 1), (2, 2), (1, 7), (3, 40), (16, 16), (33, 33), (64, 64), (100, 49), (97, 97),
+                                 (98, 98), (97, 300), (120, 120)])
+@pytest.mark.parametrize('rank', [None, 3])
+def test_truncated_svd_sizes(lib, m, c, rank):
+    """Singular values to m c eps s0 of LAPACK's, orthonormal factors, the
+    matrix back: the sizes around the lanes-per-pair steps and the largest
+    factor held in LDS (97), full rank and rank 3 (equal zero columns)."""
+    from scikit_tt_amd.utils import truncated_svd
+    gen = torch.Generator(device='cuda').manual_seed(m * 1000 + c)
+    k = min(m, c)
+    Y = _randn(gen, m, c)
+    if rank is not None:
+        Y = _randn(gen, m, rank) @ _randn(gen, rank, c)
+    u, s, v = truncated_svd(Y)
+    ref = np.linalg.svd(Y.cpu().numpy(), compute_uv=False)
+    tol = 4 * m * c * EPS * ref[0]
+    assert s.shape[0] == k and np.abs(s.cpu().numpy() - ref).max() <= tol
+    assert float(((u * s) @ v - Y).abs().max()) <= tol
+    live = min(k, rank or k)
+    for f in (u[:, :live].T, v[:live]):
+        assert float((f @ f.T - torch.eye(live, dtype=torch.float64, device='cuda')).abs().max()) <= 4 * m * c * EPS
+
+
+def test_truncated_svd_not_finite(lib):
+    """A NaN stays in the result; the kept rank stays in range."""
+    from scikit_tt_amd.utils import truncated_svd
+    Y = torch.ones((6, 5), dtype=torch.float64, device='cuda')
+    Y[2, 3] = float('nan')
+    u, s, v = truncated_svd(Y)
+    assert s.shape[0] <= 5 and bool(torch.isnan(s).any())
