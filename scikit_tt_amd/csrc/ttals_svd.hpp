@@ -34,34 +34,14 @@ __device__ __forceinline__ double lanes_sum(double v, int L) {
   return v;
 }
 
-// B (c x k, row-major, global) <- B V = U diag(sig) (orthogonal columns), V (k
-// x k, row-major, global) the rotations; sig the column norms, perm the
-// columns by decreasing norm.  lds: js_doubles(c, k).  Starts and ends with a
-// barrier.
-__device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, int* perm, double* lds_) {
-  __shared__ int s_rot[2];
-  TT_LDS double* Bl = (TT_LDS double*)lds_;
-  const int lb = c | 1, lv = k | 1;
-  TT_LDS double* Vl = Bl + k * lb;
-  TT_LDS double* sg = Vl + k * lv;
-  __syncthreads();
-  for (int e = threadIdx.x; e < c * k; e += NT) {
-    const int i = e / k, j = e - i * k;
-    Bl[j * lb + i] = B[e];
-  }
-  for (int e = threadIdx.x; e < k * lv; e += NT) {
-    const int j = e / lv, i = e - j * lv;
-    Vl[e] = i == j ? 1.0 : 0.0;
-  }
-  if (threadIdx.x < 2) s_rot[threadIdx.x] = 0;
+// Sweeps of rotations over all column pairs of Bl (k columns, c rows, ld lb)
+// and Vl (k rows, ld lv) until a sweep rotates nothing (at most 60): RM entries
+// of a column per lane, L lanes per pair (RM * L >= c, k).
+template <int RM>
+__device__ __forceinline__ void js_sweeps(TT_LDS double* Bl, TT_LDS double* Vl, int c, int k, int lb, int lv, int L,
+                                          int* s_rot) {
   const int kk = (k & 1) ? k + 1 : k, pairs = kk / 2, mod = kk - 1;
-  const int rows = c > k ? c : k;
-  int L = 8;
-  while (rows > L * JS_ROWS) L <<= 1;
-  while (L < 64 && 2 * L * pairs <= NT) L <<= 1;
-  L = __builtin_amdgcn_readfirstlane(L);
   const int l = threadIdx.x & (L - 1), g = threadIdx.x / L, ng = NT / L;
-  __syncthreads();
   for (int sweep = 0; sweep < 60; ++sweep) {
     const int flag = sweep & 1;
     for (int round = 0; round < mod; ++round) {
@@ -74,17 +54,24 @@ __device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, i
         p1 = 1 + p1;
         const int i = p0 < p1 ? p0 : p1, j = p0 < p1 ? p1 : p0;
         if (j >= k) continue;  // dummy partner
-        TT_LDS double *ci = Bl + i * lb, *cj = Bl + j * lb;
-        double bi[JS_ROWS], bj[JS_ROWS];
+        TT_LDS double *ci = Bl + i * lb, *cj = Bl + j * lb, *wi = Vl + i * lv, *wj = Vl + j * lv;
+        // the entries of V travel with those of B: their latency is off the chain
+        double bi[RM], bj[RM], vi[RM], vj[RM];
 #pragma unroll
-        for (int u = 0; u < JS_ROWS; ++u) {
+        for (int u = 0; u < RM; ++u) {
           const int r = l + u * L;
           bi[u] = r < c ? ci[r] : 0.0;
           bj[u] = r < c ? cj[r] : 0.0;
         }
+#pragma unroll
+        for (int u = 0; u < RM; ++u) {
+          const int r = l + u * L;
+          vi[u] = r < k ? wi[r] : 0.0;
+          vj[u] = r < k ? wj[r] : 0.0;
+        }
         double aii = 0.0, ajj = 0.0, aij = 0.0;
 #pragma unroll
-        for (int u = 0; u < JS_ROWS; ++u) {
+        for (int u = 0; u < RM; ++u) {
           aii = fma(bi[u], bi[u], aii);
           ajj = fma(bj[u], bj[u], ajj);
           aij = fma(bi[u], bj[u], aij);
@@ -93,19 +80,12 @@ __device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, i
         ajj = lanes_sum(ajj, L);
         aij = lanes_sum(aij, L);
         if (fabs(aij) <= 1e-15 * sqrt(aii * ajj) || aij == 0.0) continue;
-        TT_LDS double *wi = Vl + i * lv, *wj = Vl + j * lv;
-        double vi[JS_ROWS], vj[JS_ROWS];
+        // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)) for zeta = d / h: one root and one division
+        const double d = ajj - aii, h = 2.0 * aij;
+        const double t = (d >= 0.0 ? h : -h) / (fabs(d) + sqrt(fma(d, d, h * h)));
+        const double cs = 1.0 / sqrt(fma(t, t, 1.0)), sn = cs * t;
 #pragma unroll
-        for (int u = 0; u < JS_ROWS; ++u) {
-          const int r = l + u * L;
-          vi[u] = r < k ? wi[r] : 0.0;
-          vj[u] = r < k ? wj[r] : 0.0;
-        }
-        const double zeta = (ajj - aii) / (2.0 * aij);
-        const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-        const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
-#pragma unroll
-        for (int u = 0; u < JS_ROWS; ++u) {
+        for (int u = 0; u < RM; ++u) {
           const int r = l + u * L;
           if (r < c) {
             ci[r] = cs * bi[u] - sn * bj[u];
@@ -125,6 +105,50 @@ __device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, i
     __syncthreads();
     if (rot == 0) break;
   }
+}
+
+// B (c x k, row-major, global) <- B V = U diag(sig) (orthogonal columns), V (k
+// x k, row-major, global) the rotations; sig the column norms, perm the
+// columns by decreasing norm.  lds: js_doubles(c, k).  B is scaled by a power
+// of two (exactly) while it is worked on, so that the squares of its norms
+// neither overflow nor vanish.  Starts and ends with a barrier.
+__device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, int* perm, double* lds_) {
+  __shared__ int s_rot[2];
+  __shared__ double s_mx[NWAVE];
+  TT_LDS double* Bl = (TT_LDS double*)lds_;
+  const int lb = c | 1, lv = k | 1;
+  TT_LDS double* Vl = Bl + k * lb;
+  TT_LDS double* sg = Vl + k * lv;
+  __syncthreads();
+  double mx = 0.0;
+  for (int e = threadIdx.x; e < c * k; e += NT) mx = fmax(mx, fabs(B[e]));
+  mx = wave_max(mx);
+  if ((threadIdx.x & 63) == 0) s_mx[threadIdx.x >> 6] = mx;
+  if (threadIdx.x < 2) s_rot[threadIdx.x] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NWAVE; ++q) mx = fmax(mx, s_mx[q]);
+  const int ex = (mx > 0.0 && isfinite(mx)) ? -ilogb(mx) : 0;  // applied in two halves: 2^ex itself may overflow
+  const double up0 = ldexp(1.0, ex / 2), up1 = ldexp(1.0, ex - ex / 2);
+  const double dn0 = ldexp(1.0, -(ex / 2)), dn1 = ldexp(1.0, ex / 2 - ex);
+  for (int e = threadIdx.x; e < c * k; e += NT) {
+    const int i = e / k, j = e - i * k;
+    Bl[j * lb + i] = B[e] * up0 * up1;
+  }
+  for (int e = threadIdx.x; e < k * lv; e += NT) {
+    const int j = e / lv, i = e - j * lv;
+    Vl[e] = i == j ? 1.0 : 0.0;
+  }
+  const int rows = c > k ? c : k, pairs = (k + 1) / 2;
+  int L = 8;
+  while (rows > L * JS_ROWS) L <<= 1;
+  while (L < 64 && 2 * L * pairs <= NT) L <<= 1;
+  L = __builtin_amdgcn_readfirstlane(L);
+  __syncthreads();
+  if (rows <= 2 * L) js_sweeps<2>(Bl, Vl, c, k, lb, lv, L, s_rot);
+  else if (rows <= 4 * L) js_sweeps<4>(Bl, Vl, c, k, lb, lv, L, s_rot);
+  else if (rows <= 8 * L) js_sweeps<8>(Bl, Vl, c, k, lb, lv, L, s_rot);
+  else js_sweeps<JS_ROWS>(Bl, Vl, c, k, lb, lv, L, s_rot);
   // column norms (a non-finite one sorts first) and ranks by decreasing norm
   for (int j = threadIdx.x; j < k; j += NT) {
     double s0 = 0.0, s1 = 0.0;
@@ -134,7 +158,7 @@ __device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, i
     }
     if (c & 1) s0 = fma(Bl[j * lb + c - 1], Bl[j * lb + c - 1], s0);
     const double s = sqrt(s0 + s1);
-    sig[j] = s;
+    sig[j] = s * dn0 * dn1;
     sg[j] = s == s ? s : INFINITY;
   }
   __syncthreads();
@@ -146,7 +170,7 @@ __device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, i
   }
   for (int e = threadIdx.x; e < c * k; e += NT) {
     const int i = e / k, j = e - i * k;
-    B[e] = Bl[j * lb + i];
+    B[e] = Bl[j * lb + i] * dn0 * dn1;
   }
   for (int e = threadIdx.x; e < k * k; e += NT) {
     const int i = e / k, j = e - i * k;

@@ -119,6 +119,17 @@ def test_truncated_svd_sizes(lib, m, c, rank):
         assert float((f @ f.T - torch.eye(live, dtype=torch.float64, device='cuda')).abs().max()) <= 4 * m * c * EPS
 
 
+@pytest.mark.parametrize('scale', [1e-200, 1e200])
+def test_truncated_svd_scale(lib, scale):
+    """Entries whose squares leave the range of a double."""
+    from scikit_tt_amd.utils import truncated_svd
+    gen = torch.Generator(device='cuda').manual_seed(5)
+    Y = _randn(gen, 24, 24).triu()  # its QR needs no reflections: the SVD alone is at stake
+    u, s, v = truncated_svd(Y * scale)
+    ref = np.linalg.svd(Y.cpu().numpy(), compute_uv=False)
+    assert np.abs(s.cpu().numpy() / scale - ref).max() <= 4 * 24 * 24 * EPS * ref[0]
+
+
 def test_truncated_svd_not_finite(lib):
     """A NaN stays in the result; the kept rank stays in range."""
     from scikit_tt_amd.utils import truncated_svd
