@@ -28,13 +28,12 @@ using namespace ttals;
 #define TTALS_ALS_WAVES_PER_EU 2  // two resident systems per CU
 #endif
 
-// One workgroup per system (als_block).
-template <class ACC>
+// One workgroup per system (als_block); KIND 0: sle, 1: evp.
+template <int KIND>
 __global__ __launch_bounds__(NT, TTALS_ALS_WAVES_PER_EU) void k_als(const SysDesc* descs, long arena) {
-  static_assert(sizeof(ACC) == 8, "the engine computes in FP64");
   extern __shared__ double dyn_lds[];
   __shared__ SolveLDS S;
-  als_block(descs[blockIdx.x], dyn_lds, arena, S);
+  als_block<KIND>(descs[blockIdx.x], dyn_lds, arena, S);
 }
 
 struct PieceArgs {
@@ -62,7 +61,7 @@ enum PieceOp { P_LEFT_OP, P_RIGHT_OP, P_LEFT_RHS, P_RIGHT_RHS, P_MICRO_DENSE, P_
 // One workgroup.  The matvec, local solve and local eigensolve take the
 // engine's on-chip path (operator and working vectors in the dynamic LDS
 // arena) whenever the problem fits `A.arena`, else the global path.
-__global__ __launch_bounds__(NT) void k_piece(PieceArgs A) {
+__global__ __launch_bounds__(NT, TTALS_ALS_WAVES_PER_EU) void k_piece(PieceArgs A) {
   __shared__ double lds[GEMM_LDS_DOUBLES];
   __shared__ SolveLDS S;
   extern __shared__ double dyn_lds[];
@@ -131,7 +130,9 @@ __global__ __launch_bounds__(NT) void k_piece(PieceArgs A) {
       int its = 0, r = 0;
       int method = A.method;
       if (method == 0) method = (N <= NDENSE) ? 1 : (A.sym ? 2 : 3);
-      if (method == 1) {
+      if (method == 1 && lu_reg_fits(A.a, A.P, A.n, A.Q, A.b, A.arena)) {
+        r = lu_reg_solve(A.a, A.P, A.n, A.Q, A.b, A.L, A.A, A.R, A.f, A.v, dyn_lds) ? 0 : 1;
+      } else if (method == 1) {
         micro_dense<double>(A.a, A.P, A.n, A.Q, A.b, A.L, A.A, A.R, A.V, N);
         wg_copy(A.f, A.v, N);
         __syncthreads();
@@ -1293,7 +1294,7 @@ int enqueue_batch(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, Placemen
     if (!c->k1) HIPCHK(c, hipEventCreate(&c->k1));
     HIPCHK(c, hipEventRecord(c->k0, stream));
   }
-  hipLaunchKernelGGL(k_als<double>, dim3(count), dim3(NT), (size_t)arena * 8, stream,
+  hipLaunchKernelGGL(kind == 0 ? k_als<0> : k_als<1>, dim3(count), dim3(NT), (size_t)arena * 8, stream,
                      (const SysDesc*)dptr(m_descs), arena);
   HIPCHK(c, hipGetLastError());
   if (timed) {

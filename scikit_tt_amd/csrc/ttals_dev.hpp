@@ -21,6 +21,15 @@ constexpr int NT = TTALS_NT;
 constexpr int NWAVE = NT / 64;
 static_assert(NT == 256 || NT == 512, "the tile shapes below assume 4 or 8 waves");
 
+// f(0), ..., f(N - 1) with the index a compile-time constant (register arrays)
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // index maps: a matrix row (or column) index i is split into
 // (i / div, i % div) and mapped to  (i / div) * hi + (i % div) * lo.

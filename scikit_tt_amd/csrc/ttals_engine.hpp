@@ -3,11 +3,12 @@
 // `count` workgroups solves `count` independent systems of uneven order and
 // rank; the plain drop-in path is the same kernel with count = 1.
 #pragma once
+#include "ttals_lu.hpp"
 #include "ttals_solve.hpp"
 
 namespace ttals {
 
-constexpr int NDENSE = 96;  // local systems up to this size use dense LU
+constexpr int NDENSE = LU_MAX;  // local systems up to this size use dense LU
 
 enum Status : int {
   ST_OK = 0,
@@ -198,12 +199,12 @@ __device__ __forceinline__ double fl_qr(double m, double c) {
 // arena, they are staged in LDS and contracted with ds_gemm; otherwise the
 // global-memory path (wg_gemm) runs.
 
-template <class ACC>
+template <class ACC, int KIND>
 __device__ double build_left(int i, const SysDesc& D, ACC* lds, long cap) {
   // L_i from L_{i-1} and core i-1
   const int j = i - 1;
   const int a = D.rx[j], n = D.n[j], b = D.rx[i], P = D.ra[j], Q = D.ra[i];
-  const bool rhs = (D.kind == 0);
+  constexpr bool rhs = KIND == 0;
   const int p = D.rb[j], q = D.rb[i];
   const double fl = fl_op(a, P, n, Q, b) + (rhs ? fl_rhs(a, p, n, q, b) : 0.0);
   const long t1n = rhs && (long)a * n * q > ds_t1_size(a, P, n, b) ? (long)a * n * q : ds_t1_size(a, P, n, b);
@@ -244,13 +245,13 @@ __device__ double build_left(int i, const SysDesc& D, ACC* lds, long cap) {
   return fl;
 }
 
-template <class ACC>
+template <class ACC, int KIND>
 __device__ double build_right(int i, const SysDesc& D, ACC* lds, long cap) {
   // R_i from R_{i+1} and core i+1: the left-form update of the mirrored
   // problem (ranks a <-> b, operator ranks P <-> Q)
   const int j = i + 1;
   const int a = D.rx[j], n = D.n[j], b = D.rx[j + 1], P = D.ra[j], Q = D.ra[j + 1];
-  const bool rhs = (D.kind == 0);
+  constexpr bool rhs = KIND == 0;
   const int p = D.rb[j], q = D.rb[j + 1];
   const double fl = fl_op(a, P, n, Q, b) + (rhs ? fl_rhs(a, p, n, q, b) : 0.0);
   const long t1n = rhs && (long)a * n * q > ds_t1_size(b, Q, n, a) ? (long)a * n * q : ds_t1_size(b, Q, n, a);
@@ -328,8 +329,9 @@ __host__ __device__ __forceinline__ long arena_need_onchip(int a, int P, int n, 
   const long n2 = arena_need_m2(a, P, n, Q, b, nvec);
   return n2 < n3 ? n2 : n3;
 }
+template <int KIND>
 __device__ __forceinline__ long arena_need(const SysDesc& D, int a, int P, int n, int Q, int b) {
-  return arena_need_onchip(a, P, n, Q, b, D.kind == 0 ? 5 : 3, D.mvar);
+  return arena_need_onchip(a, P, n, Q, b, KIND == 0 ? 5 : 3, D.mvar);
 }
 
 // Sets up the on-chip local operator of `op` in the arena `ar` (`cap`
@@ -389,7 +391,7 @@ __device__ __forceinline__ void onchip_work(Work& W, double* vec, int N, bool sl
 // next position into D.g.  Returns a Status.  `lds` is the dynamic LDS
 // region: GEMM staging tiles, or (during a local solve that fits) the
 // on-chip arena of `arena` doubles.
-template <class ACC>
+template <class ACC, int KIND>
 __device__ int local_step(int i, bool forward, const SysDesc& D, bool sym, ACC* lds, long arena, SolveLDS& S,
                           double* lam, StepStats& st) {
   const int a = D.rx[i], n = D.n[i], b = D.rx[i + 1];
@@ -398,9 +400,9 @@ __device__ int local_step(int i, bool forward, const SysDesc& D, bool sym, ACC* 
   LocalOp<double> op{a, P, n, Q, b, D.Ls + D.Loff[i], D.ac[i], D.Rs + D.Roff[i], D.t1, D.t2, false};
   int its = 0;
   const double fmv = fl_op(a, P, n, Q, b);
-  const bool dense = (D.kind == 0 && N <= NDENSE);
+  const bool dense = (KIND == 0 && N <= NDENSE);
   if (threadIdx.x == 0) S.vfl = 0.0;  // vector flops of this local solve, counted by the solvers
-  if (D.kind == 0) {
+  if constexpr (KIND == 0) {
     st.flops += fl_rhs(a, D.rb[i], n, D.rb[i + 1], b);
     micro_rhs<double, ACC>(a, D.rb[i], n, D.rb[i + 1], b, D.Lbs + D.Lboff[i], D.bc[i], D.Rbs + D.Rboff[i], D.f,
                            D.t1, lds);
@@ -409,11 +411,11 @@ __device__ int local_step(int i, bool forward, const SysDesc& D, bool sym, ACC* 
   const long long tsetup = ph_now();
   Work W;
   W.V = D.V;
-  const bool onchip = !dense && arena_need(D, a, P, n, Q, b) <= arena;
+  const bool onchip = !dense && arena_need<KIND>(D, a, P, n, Q, b) <= arena;
   if (onchip) {
-    double* vec = onchip_operator(op, reinterpret_cast<double*>(lds), arena, D.kind == 0 ? 5 : 3, D.mvar);
-    onchip_work(W, vec, N, D.kind == 0);
-    if (D.kind == 0) {
+    double* vec = onchip_operator(op, reinterpret_cast<double*>(lds), arena, KIND == 0 ? 5 : 3, D.mvar);
+    onchip_work(W, vec, N, KIND == 0);
+    if constexpr (KIND == 0) {
       wg_copy(D.f, W.f, N);
       wg_copy(D.g, W.x, N);
     }
@@ -423,20 +425,25 @@ __device__ int local_step(int i, bool forward, const SysDesc& D, bool sym, ACC* 
     W.x = D.g;
     // sle: CG vectors in the (then unused) basis area; evp: Lanczos' previous
     // vector in the rhs buffer, which evp does not use
-    W.r = (D.kind == 0) ? D.V : D.f;
+    W.r = (KIND == 0) ? D.V : D.f;
     W.p = D.V + N;
     W.q = D.V + 2 * (long)N;
     W.cur = D.qw;
     W.w = D.qq;
   }
   ph_add(S, PH_SETUP, tsetup);
-  if (D.kind == 0) {
+  if constexpr (KIND == 0) {
     if (dense) {
-      micro_dense<double>(a, P, n, Q, b, op.L, op.A, op.R, D.dense, N);
-      wg_copy(D.f, D.g, N);
-      __syncthreads();
-      int* piv = reinterpret_cast<int*>(D.dense + (long)NDENSE * NDENSE);
-      if (!wg_lu_solve(D.dense, N, D.g, piv, S.red)) return ST_SINGULAR;
+      if (lu_reg_fits(a, P, n, Q, b, arena)) {
+        if (!lu_reg_solve(a, P, n, Q, b, op.L, op.A, op.R, D.f, D.g, reinterpret_cast<double*>(lds)))
+          return ST_SINGULAR;
+      } else {  // more unknowns, or operator pieces that do not fit the arena: the matrix in global memory
+        micro_dense<double>(a, P, n, Q, b, op.L, op.A, op.R, D.dense, N);
+        wg_copy(D.f, D.g, N);
+        __syncthreads();
+        int* piv = reinterpret_cast<int*>(D.dense + (long)NDENSE * NDENSE);
+        if (!wg_lu_solve(D.dense, N, D.g, piv, S.red)) return ST_SINGULAR;
+      }
       st.flops += 3.0 * (double)N * N * P * Q + (2.0 / 3.0) * (double)N * N * N + 2.0 * (double)N * N;
       // the operator pieces read once, the micro matrix written and read once
       st.mvb += by_op(a, P, n, Q, b, 8.0, false) + 8.0 * (2.0 * (double)N * N - N);
@@ -493,7 +500,7 @@ __device__ int local_step(int i, bool forward, const SysDesc& D, bool sym, ACC* 
     t[5] = st.last_res;
   }
   ++st.nsolve;
-  if (D.kind == 0) {  // (the eigensolver checks its Ritz vector itself)
+  if constexpr (KIND == 0) {  // (the eigensolver checks its Ritz vector itself)
     const double nv = wg_nrm2(D.g, N, S.red);
     if (!isfinite(nv)) return ST_NONFINITE;
   }
@@ -655,7 +662,9 @@ __device__ double operator_asymmetry(const SysDesc& D, SolveLDS& S) {
   return sqrt(fmax(0.0, 2.0 * (1.0 - at / aa)));
 }
 
-template <class ACC>
+// KIND 0: sle, 1: evp -- one kernel each, so that neither allocates registers
+// and instruction cache for the other's solvers.
+template <class ACC, int KIND>
 __device__ void als_solve(const SysDesc& D, ACC* lds, long arena, SolveLDS& S) {
   const int d = D.d;
   if (threadIdx.x < 8) S.prof[threadIdx.x] = 0;
@@ -677,28 +686,28 @@ __device__ void als_solve(const SysDesc& D, ACC* lds, long arena, SolveLDS& S) {
   // evp's local eigensolver (Lanczos) needs a symmetric operator: one whose
   // slices are not symmetric one by one is checked as a whole and rejected
   // when it is not symmetric (the reference's 'eig' would call dgeev)
-  if (D.kind == 1 && !sym) {
+  if (KIND == 1 && !sym) {
     if (operator_asymmetry(D, S) > SYM_TOL) status = ST_NONSYM;
   }
 
-  if (D.kind == 0 && D.ortho_x0) ortho_right_x<ACC>(D, lds, arena, S);
+  if (KIND == 0 && D.ortho_x0) ortho_right_x<ACC>(D, lds, arena, S);
 
   // boundary stacks
   set_one(D.Ls + D.Loff[0]);
   set_one(D.Rs + D.Roff[d - 1]);
-  if (D.kind == 0) {
+  if constexpr (KIND == 0) {
     set_one(D.Lbs + D.Lboff[0]);
     set_one(D.Rbs + D.Rboff[d - 1]);
   }
   __syncthreads();
   if (status == ST_OK)
-    for (int i = d - 2; i >= 0; --i) st.flops += build_right<ACC>(i, D, lds, arena);
+    for (int i = d - 2; i >= 0; --i) st.flops += build_right<ACC, KIND>(i, D, lds, arena);
 
   bool converged = false;
   double lam1 = 0.0, lam2 = 0.0;  // eigenvalue after the last and the second-to-last sweep
   st.tol = D.tol;
   while (sweeps < D.repeats && !converged && status == ST_OK) {
-    if (D.kind == 1 && D.adapt) {
+    if (KIND == 1 && D.adapt) {
       // Inexact ALS: the local eigenproblems need only be solved to the
       // accuracy the sweep itself has reached.  The eigenvalue error of a
       // Lanczos pair with residual r is O(r^2), so the tolerance follows the
@@ -713,33 +722,33 @@ __device__ void als_solve(const SysDesc& D, ACC* lds, long arena, SolveLDS& S) {
     __syncthreads();
     for (int i = 0; i < d && status == ST_OK; ++i) {
       const long long ts = ph_now();
-      if (i > 0) st.flops += build_left<ACC>(i, D, lds, arena);
+      if (i > 0) st.flops += build_left<ACC, KIND>(i, D, lds, arena);
       ph_add(S, PH_STACK, ts);
       if (i < d - 1) {
         if (over_budget(D.budget, t_begin, &S.flag[3])) {
           status = ST_DEADLINE;
           break;
         }
-        status = local_step<ACC>(i, true, D, sym, lds, arena, S, &lam, st);
+        status = local_step<ACC, KIND>(i, true, D, sym, lds, arena, S, &lam, st);
         ++nsolves;
       }
     }
     for (int i = d - 1; i >= 0 && status == ST_OK; --i) {
       const long long ts = ph_now();
-      if (i < d - 1) st.flops += build_right<ACC>(i, D, lds, arena);
+      if (i < d - 1) st.flops += build_right<ACC, KIND>(i, D, lds, arena);
       ph_add(S, PH_STACK, ts);
       if (over_budget(D.budget, t_begin, &S.flag[3])) {
         status = ST_DEADLINE;
         break;
       }
-      status = local_step<ACC>(i, false, D, sym, lds, arena, S, &lam, st);
+      status = local_step<ACC, KIND>(i, false, D, sym, lds, arena, S, &lam, st);
       ++nsolves;
     }
     if (status != ST_OK) break;
     ++sweeps;
     lam2 = lam1;
     lam1 = lam;
-    if (D.kind == 1) {
+    if constexpr (KIND == 1) {
       // best-so-far pair (strict improvement in |lambda - sigma|), then the
       // convergence test over the last <= 3 sweeps
       if (fabs(lam - D.sigma) < fabs(best - D.sigma)) {
@@ -756,7 +765,7 @@ __device__ void als_solve(const SysDesc& D, ACC* lds, long arena, SolveLDS& S) {
       ++nhist;
     }
   }
-  if (D.kind == 1 && status == ST_OK && sweeps > 0) {
+  if (KIND == 1 && status == ST_OK && sweeps > 0) {
     for (int i = 0; i < d; ++i) wg_copy(D.bestc[i], D.xc[i], D.best_rx[i] * D.n[i] * D.best_rx[i + 1]);
     for (int i = threadIdx.x; i <= d; i += NT) D.rx[i] = D.best_rx[i];
     lam = best;
@@ -782,6 +791,7 @@ __device__ void als_solve(const SysDesc& D, ACC* lds, long arena, SolveLDS& S) {
 // One workgroup per system.  Dynamic LDS (`arena` doubles, at least the
 // GEMM staging tiles) holds either the staging tiles or the on-chip copy of
 // a local problem.
+template <int KIND>
 __device__ __forceinline__ void als_block(const SysDesc& D, double* dyn_lds, long arena, SolveLDS& S) {
   // x <- x0: the engine works in place on the output cores
   for (int i = 0; i < D.d; ++i) {
@@ -792,7 +802,7 @@ __device__ __forceinline__ void als_block(const SysDesc& D, double* dyn_lds, lon
     for (long e = threadIdx.x; e < len; e += NT) dst[e] = src[e];
   }
   __syncthreads();
-  als_solve<double>(D, dyn_lds, arena, S);
+  als_solve<double, KIND>(D, dyn_lds, arena, S);
   __syncthreads();
   // one compact row per system, so the host fetches every result with one copy
   for (int k = threadIdx.x; k < RES_HEAD + 1 + D.d; k += NT) D.res[k] = k < RES_HEAD ? D.out[k] : (double)D.rx[k - RES_HEAD];

@@ -26,7 +26,7 @@ __global__ __launch_bounds__(NT) void k_hybrid(const GangDesc* gdescs, const int
   if (blk < gang_blocks)
     gang_block(gdescs, block_sys, blk, dyn_lds, arena, S);
   else
-    als_block(descs[blk - gang_blocks], dyn_lds, arena, S);
+    als_block<0>(descs[blk - gang_blocks], dyn_lds, arena, S);
 }
 
 hipError_t hybrid_occupancy(int* per_cu, size_t dyn_lds) {

@@ -97,14 +97,6 @@ __device__ __forceinline__ T* uni(T* p) {
   return reinterpret_cast<T*>(((unsigned long)hi << 32) | lo);
 }
 
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
-
 // A block's columns in registers: rows [w RW, (w+1) RW) of the `rows` below
 // (and with) the block's first pivot row; b[s] = row w RW + 4 s + lk, column li.
 template <int RP>

@@ -137,3 +137,32 @@ def test_truncated_svd_not_finite(lib):
     Y[2, 3] = float('nan')
     u, s, v = truncated_svd(Y)
     assert s.shape[0] <= 5 and bool(torch.isnan(s).any())
+
+
+# (a, P, n, Q, b): local sizes around the lane, wave and row-half edges of the register LU (1 .. 96 unknowns)
+LOCAL = [(1, 1, 1, 1, 1), (1, 2, 3, 1, 1), (2, 3, 4, 2, 2), (1, 1, 31, 1, 1), (2, 2, 4, 2, 4), (3, 1, 11, 2, 1),
+         (4, 3, 4, 3, 4), (5, 2, 13, 1, 1), (4, 2, 4, 2, 6), (5, 1, 19, 1, 1), (1, 2, 2, 4, 48)]
+
+
+@pytest.mark.parametrize('kb', [61, 0])
+@pytest.mark.parametrize('a,P,n,Q,b', LOCAL)
+def test_local_lu(lib, a, P, n, Q, b, kb):
+    """Dense local solve against LAPACK, in registers and (no arena) in global
+    memory; the residual of LU with partial pivoting is below N^2 eps |M| |v|
+    for these sizes and growth factors."""
+    from scikit_tt_amd import _lib
+    gen = torch.Generator(device='cuda').manual_seed(a * 100 + b)
+    L, A, R = _randn(gen, a, P, a), _randn(gen, P, n, n, Q), _randn(gen, b, Q, b)
+    N = a * n * b
+    f, v = _randn(gen, N), _randn(gen, N)
+    M = torch.tensordot(torch.tensordot(L, A, dims=([1], [0])), R, dims=([4], [1])).permute(1, 2, 5, 0, 3, 4).reshape(N, N)
+    ctx = _lib.context(0)
+    assert lib.ttals_set_arena_kb(ctx, kb) == 0
+    try:
+        its = ctypes.c_int()
+        assert lib.ttals_local_solve(ctx, None, a, P, n, Q, b, _ptr(L), _ptr(A), _ptr(R), _ptr(f), _ptr(v), 1, 0, 1e-12,
+                                     100, ctypes.byref(its)) == 0
+    finally:
+        assert lib.ttals_set_arena_kb(ctx, 61) == 0
+    res = float((M @ v - f).norm())
+    assert res <= 4 * N * N * EPS * float(M.norm()) * float(v.norm())
