@@ -4,6 +4,7 @@
 // rank; the plain drop-in path is the same kernel with count = 1.
 #pragma once
 #include "ttals_lu.hpp"
+#include "ttals_qr.hpp"
 #include "ttals_solve.hpp"
 
 namespace ttals {
@@ -92,9 +93,8 @@ __device__ __forceinline__ void set_one(double* p) {
 }
 
 // Buffers of one QR: W (m x c), Q (m x k), R (k x c), tau (k).  With `lds`
-// set (global-memory panels: the arena is free), a tall panel is factored by
-// the blocked Householder QR: lds / lds_cap its LDS, tws its global T
-// storage.
+// set (global-memory panels: the arena is free), the panel is factored by a
+// blocked Householder QR: lds / lds_cap its LDS, tws its global T storage.
 struct QRBuf {
   double* W;
   double* Q;
@@ -105,13 +105,15 @@ struct QRBuf {
   double* tws = nullptr;
 };
 
-// On-chip QR buffers carved from the arena when m x c fits, else the global
-// scratch of the system (then the arena is free for the blocked QR's block,
-// and its T storage is the dense-LU buffer, which no QR overlaps).
+// On-chip QR buffers carved from the arena when the panel fits and is a small
+// one (the register QR, or a column sweep of at most 8 columns: about 3.5 us a
+// column in LDS, where a block of 16 columns costs the blocked QR 30 us), else
+// the global scratch of the system (then the arena is free for the blocked
+// QR's block, and its T storage is the dense-LU buffer, which no QR overlaps).
 __device__ __forceinline__ QRBuf qr_buffers(const SysDesc& D, int m, int c, double* arena, long cap) {
   const long k = m < c ? m : c;
   const long need = (long)m * c + (long)m * k + k * c + k;
-  if (need <= cap) return QRBuf{arena, arena + (long)m * c, arena + (long)m * c + (long)m * k,
+  if (need <= cap && ((m <= 64 && c <= 64) || c <= 8)) return QRBuf{arena, arena + (long)m * c, arena + (long)m * c + (long)m * k,
                                  arena + (long)m * c + (long)m * k + k * c};
   QRBuf B{D.qw, D.qq, D.rf, D.tau};
   if (cap >= GEMM_LDS_DOUBLES && ((long)c + 16) * 16 <= (long)NDENSE * NDENSE) {
@@ -148,14 +150,24 @@ __device__ __forceinline__ void qr_load_panel(double* W, const double* v, int m,
 // v is (m x c) row-major (forward) or (c x m) row-major transposed
 // (backward).  Householder QR of the (m x c) view: explicit Q (m x k) into
 // B.Q, the clean upper-triangular R (k x c) into B.R.  Returns k.  Small
-// panels: the register QR (wg_qr_small); tall global-memory panels: the
-// blocked form (wg_hhqr_blocked); else the column sweep.
+// panels: the register QR (wg_qr_small); global-memory panels: the blocked
+// QR with its block in registers (wg_hqr, up to HQ_ROWS_MAX rows), above that
+// the one with its block in LDS (wg_hhqr_blocked); else the column sweep.
 __device__ int qr_factor(const double* v, int m, int c, bool transposed, const QRBuf& B, SolveLDS& S) {
   double* W = B.W;
   qr_load_panel(W, v, m, c, transposed);
   const int k = m < c ? m : c;
   if (m <= 64 && c <= 64) {
     wg_qr_small(W, m, c, B.tau, B.Q, B.R);
+    return k;
+  }
+  if (B.lds && m <= HQ_ROWS_MAX && hq_fits(m, c) && (long)sizeof(HqLDS) <= 8 * B.lds_cap) {
+    wg_hqr(W, m, c, c, B.tws, (HqL)B.lds);
+    for (int e = threadIdx.x; e < k * c; e += NT) {
+      const int i = e / c, j = e - i * c;
+      B.R[e] = j >= i ? W[e] : 0.0;
+    }
+    wg_hqr_form_q(W, m, c, c, B.tws, B.Q, (HqL)B.lds);
     return k;
   }
   if (B.lds && wg_hhqr_blocked(W, m, c, B.Q, B.R, B.tws, B.tau, B.lds, B.lds_cap, S.red)) return k;
