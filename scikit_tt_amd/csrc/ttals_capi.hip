@@ -1409,7 +1409,7 @@ bool dims_ok(std::initializer_list<int> v) {
 // in k_als's 61 KB.  An arena the caller set is kept as is.
 int hybrid_arena(ttals_ctx* c, long* out) {
   if (c->arena_hybrid == 0) {
-    long doubles = std::max<long>(c->arena, GEMM_LDS_DOUBLES);
+    long doubles = std::max<long>(c->arena, hybrid_min_arena());
     if (!c->arena_set) {
       int max_lds = 0;
       size_t stat = 0;

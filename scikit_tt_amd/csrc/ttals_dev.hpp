@@ -1324,6 +1324,82 @@ __device__ __forceinline__ bool cholqr_small_step(double* Rp, double* Rt, double
   return true;
 }
 
+// The same step for c <= 64 with R^{-1} in a buffer of its own (Ri), all in
+// LDS.  Bound by dependent steps, so few barriers: the Cholesky factor is
+// formed in registers (lane = row, a block of columns per wave), one LDS
+// exchange of the unscaled pivot column and one barrier per column, R's row
+// written by the waves in turn off that chain; then one wave inverts R (a lane
+// per column, no barrier) while another accumulates Rt <- R Rt (likewise).
+// 48 x 48: 26 us against 170 us for cholqr_small_step, whose columns and rows
+// cost two or three barriers each.  col holds 128 doubles.
+__device__ __attribute__((noinline)) bool cholqr_wave_step(double* Rp_, double* Rt_, double* Ri_, double* col_, int c_) {
+  constexpr int CB = 64 / NWAVE;
+  TT_LDS double* Rp = (TT_LDS double*)Rp_;
+  TT_LDS double* Rt = (TT_LDS double*)Rt_;
+  TT_LDS double* Ri = (TT_LDS double*)Ri_;
+  TT_LDS double* col = (TT_LDS double*)col_;
+  const int c = __builtin_amdgcn_readfirstlane(c_);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double a[CB];  // row `lane`, columns w CB .. w CB + CB - 1
+#pragma unroll
+  for (int q = 0; q < CB; ++q) a[q] = (lane < c && w * CB + q < c) ? Rp[lane * c + w * CB + q] : 0.0;
+  bool ok = true;
+  for (int wo = 0; wo < NWAVE && ok; ++wo) {
+    static_for<0, CB>([&](auto Qc) {
+      constexpr int q = decltype(Qc)::value;
+      const int j = wo * CB + q;
+      if (j >= c || !ok) return;
+      TT_LDS double* cj = col + (j & 1) * 64;
+      if (w == wo) cj[lane] = a[q];
+      __syncthreads();
+      const double piv = cj[j], mine = cj[lane];
+      if (!(piv > 0.0) || !isfinite(piv)) {
+        ok = false;
+        return;
+      }
+      if (w >= wo) {
+        const double l = lane > j ? mine * (1.0 / piv) : 0.0;
+#pragma unroll
+        for (int u = 0; u < CB; ++u)
+          if (w > wo || u > q) a[u] -= l * cj[min(w * CB + u, 63)];
+      }
+      if (w == j % NWAVE && lane < c) Rp[j * c + lane] = lane > j ? mine / sqrt(piv) : (lane == j ? sqrt(piv) : 0.0);
+    });
+  }
+  __syncthreads();
+  if (!ok) return false;
+  if (w == 0 && lane < c) {
+    // column `lane` of R^{-1} from the bottom: x_i = -(sum_{k > i} R[i][k] x_k) / R[i][i]
+    for (int i = c - 1; i >= 0; --i) {
+      double s0 = 0.0, s1 = 0.0;
+      int k = i + 1;
+#pragma unroll 4
+      for (; k + 1 < c; k += 2) {
+        s0 += Rp[i * c + k] * Ri[k * c + lane];
+        s1 += Rp[i * c + k + 1] * Ri[(k + 1) * c + lane];
+      }
+      if (k < c) s0 += Rp[i * c + k] * Ri[k * c + lane];
+      const double d = Rp[i * c + i];
+      Ri[i * c + lane] = i > lane ? 0.0 : (i == lane ? 1.0 / d : -(s0 + s1) / d);
+    }
+  } else if (w == 1 && lane < c) {
+    // column `lane` of R Rt, row p from the rows >= p of the old one
+    for (int p = 0; p < c; ++p) {
+      double s0 = 0.0, s1 = 0.0;
+      int k = p;
+#pragma unroll 4
+      for (; k + 1 < c; k += 2) {
+        s0 += Rp[p * c + k] * Rt[k * c + lane];
+        s1 += Rp[p * c + k + 1] * Rt[(k + 1) * c + lane];
+      }
+      if (k < c) s0 += Rp[p * c + k] * Rt[k * c + lane];
+      Rt[p * c + lane] = p <= lane ? s0 + s1 : 0.0;
+    }
+  }
+  __syncthreads();
+  return true;
+}
+
 // The shift of the first shifted Cholesky QR pass for an (m x c) panel whose
 // Gram matrix has trace tr (= ||W||_F^2): 11 (m c + c (c + 1)) u tr keeps the
 // shifted Gram matrix positive definite in floating point for condition
@@ -1383,10 +1459,10 @@ __device__ __forceinline__ void row16_sum_n(double (&p)[C]) {
   for (int u = 0; u < C; ++u) p[u] += dpp_mov<0x140>(p[u]);
 }
 
-// Householder QR of a small (m x c) row-major panel W, m <= 16 R, c <= 16 C,
+// Householder QR of a small (m x c) row-major panel W, m <= 16 R, c <= DROWS C,
 // LAPACK convention (v_j = 1 at row j, H_j = I - tau_j v_j v_j^T, beta =
-// -sign(alpha) |x|).  The workgroup's 16 DPP rows (4 waves x 4 rows of 16
-// lanes) each own the columns r, r+16, ... (r = DPP row); lane l of a row
+// -sign(alpha) |x|).  The workgroup's DPP rows (4 rows of 16 lanes per wave)
+// each own the columns r, r+DROWS, ... (r = DPP row); lane l of a row
 // holds the panel rows l, l+16, ... of those columns in registers, so a
 // column's dot product is an in-register sum plus a 16-lane DPP reduction,
 // with no cross-row traffic.  Step j: column j's owner row forms the
@@ -1395,22 +1471,23 @@ __device__ __forceinline__ void row16_sum_n(double (&p)[C]) {
 // it to its later columns.  Explicit Q (m x k, ld k) goes to Qm by backward
 // accumulation in the same layout, the clean R (k x c) to Rm; W keeps the
 // reflectors.
+constexpr int DROWS = NT / 16;  // DPP rows of the workgroup
 template <int R, int C>
 __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, double* Rm) {
-  const int l16 = threadIdx.x & 15, r = threadIdx.x >> 4;  // lane in row, DPP row 0..15
+  const int l16 = threadIdx.x & 15, r = threadIdx.x >> 4;  // lane in row, DPP row
   const int k = m < c ? m : c;
   double a[R][C];
 #pragma unroll
   for (int q = 0; q < R; ++q)
 #pragma unroll
     for (int u = 0; u < C; ++u) {
-      const int i = l16 + 16 * q, jj = r + 16 * u;
+      const int i = l16 + 16 * q, jj = r + DROWS * u;
       a[q][u] = (i < m && jj < c) ? W[i * c + jj] : 0.0;
     }
   __syncthreads();  // W is rewritten column by column below
   for (int j = 0; j < k; ++j) {
-    if (r == (j & 15)) {
-      const int uj = j >> 4;
+    if (r == j % DROWS) {
+      const int uj = j / DROWS;
       double x[R];
 #pragma unroll
       for (int q = 0; q < R; ++q) {
@@ -1459,7 +1536,7 @@ __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, 
         double s = 0.0;
 #pragma unroll
         for (int q = 0; q < R; ++q) s += v[q] * a[q][u];
-        p[u] = (r + 16 * u > j) ? s : 0.0;
+        p[u] = (r + DROWS * u > j) ? s : 0.0;
       }
       row16_sum_n<C>(p);
 #pragma unroll
@@ -1475,7 +1552,7 @@ __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, 
   for (int q = 0; q < R; ++q)
 #pragma unroll
     for (int u = 0; u < C; ++u) {
-      const int i = l16 + 16 * q, jj = r + 16 * u;
+      const int i = l16 + 16 * q, jj = r + DROWS * u;
       if (jj >= k && jj < c && i < m) W[i * c + jj] = a[q][u];
     }
   __syncthreads();
@@ -1491,7 +1568,7 @@ __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, 
 #pragma unroll
   for (int q = 0; q < R; ++q)
 #pragma unroll
-    for (int u = 0; u < C; ++u) qm[q][u] = (l16 + 16 * q == r + 16 * u) ? 1.0 : 0.0;
+    for (int u = 0; u < C; ++u) qm[q][u] = (l16 + 16 * q == r + DROWS * u) ? 1.0 : 0.0;
   // reflector j-1 is read while H_j is applied
   double tn = 0.0, wn[R];
 #pragma unroll
@@ -1541,7 +1618,7 @@ __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, 
   for (int q = 0; q < R; ++q)
 #pragma unroll
     for (int u = 0; u < C; ++u) {
-      const int i = l16 + 16 * q, jj = r + 16 * u;
+      const int i = l16 + 16 * q, jj = r + DROWS * u;
       if (i < m && jj < k) Qm[i * k + jj] = qm[q][u];
     }
   __syncthreads();
@@ -1551,8 +1628,8 @@ __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, 
 __device__ void wg_qr_small(double* W, int m, int c, double* tau, double* Qm, double* Rm) {
   if (m <= 16 && c <= 16) wg_qr_small_t<1, 1>(W, m, c, tau, Qm, Rm);
   else if (m <= 32 && c <= 16) wg_qr_small_t<2, 1>(W, m, c, tau, Qm, Rm);
-  else if (m <= 32 && c <= 32) wg_qr_small_t<2, 2>(W, m, c, tau, Qm, Rm);
-  else wg_qr_small_t<4, 4>(W, m, c, tau, Qm, Rm);
+  else if (m <= 32 && c <= 32) wg_qr_small_t<2, 32 / DROWS>(W, m, c, tau, Qm, Rm);
+  else wg_qr_small_t<4, 64 / DROWS>(W, m, c, tau, Qm, Rm);
 }
 
 // Explicit Q (m x k, row-major, ld = k) from the reflectors in W.

@@ -252,7 +252,7 @@ __device__ void wg_gemm_skinny(int M, int N, int K, CView<T> A, const T* B, int 
 // y[a', m, b'] for a' in [r0, r1) of the local matvec (all three stages
 // for those rows; v read whole).  t1, t2: this member's scratch.
 template <class T>
-__device__ void gang_matvec(int a, int P, int n, int Q, int b, const T* L, const T* Ac, const T* R, const T* v,
+__device__ TT_COLD void gang_matvec(int a, int P, int n, int Q, int b, const T* L, const T* Ac, const T* R, const T* v,
                             T* y, int r0, int r1, T* t1, T* t2, T* lds) {
   const int s = r1 - r0;
   if (s <= 0) return;
@@ -274,7 +274,7 @@ __device__ void gang_matvec(int a, int P, int n, int Q, int b, const T* L, const
 //   Lout[b, Q, b'] = sum L[a, P, a'] x[a, n, b] A[P, m, n, Q] x[a', m, b']
 // (scikit_tt/solvers/sle.py:214-219).  A right stack is the same update of
 // the mirrored problem.
-__device__ void gang_stack_left(int a, int P, int n, int Q, int b, const double* L, const double* Ac,
+__device__ TT_COLD void gang_stack_left(int a, int P, int n, int Q, int b, const double* L, const double* Ac,
                                 const double* x, double* Lout, int c0, int c1, double* t1, double* t2,
                                 double* lds) {
   const int sb = c1 - c0;
@@ -363,7 +363,7 @@ __device__ __forceinline__ GangLocal gang_local(const GangCtx& C, int i) {
 // matvec on operands (L, A, R) of type T, reductions in FP64.  Returns 0
 // converged, 1 p^T M p <= 0 (not SPD), 2 maxit, -1 gang aborted.
 template <class T>
-__device__ int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R, T* x, const T* f, T* r,
+__device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R, T* x, const T* f, T* r,
                        T* p, T* q, double tol, int maxit, int* iters, double* vfl) {
   const int G = C.G, g = C.g;
   const int ld = GANG_LD;
@@ -440,7 +440,7 @@ __device__ int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const T* A, c
 // residual of an orthonormal basis is the true one to rounding) and counts
 // it in *unconfirmed.
 template <class T>
-__device__ int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R, T* x, const T* f,
+__device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R, T* x, const T* f,
                           T* w, T* V, double tol, int maxit, int m, int* iters, double* vfl, int* unconfirmed) {
   const int G = C.G, g = C.g;
   const int ld = GANG_LD;
@@ -658,7 +658,7 @@ __device__ double gang_build_left(GangCtx& C, int i) {
 // R_i from R_{i+1} and core i+1: the transposed core and operator core are
 // written first (split), then the left update of the mirrored problem
 // (rows a of the output); member 0 also the rhs stack.  Two barriers.
-__device__ double gang_build_right(GangCtx& C, int i, bool* ok) {
+__device__ TT_COLD double gang_build_right(GangCtx& C, int i, bool* ok) {
   const GangDesc& D = C.D;
   const int j = i + 1;
   const int a = D.rx[j], n = D.n[j], b = D.rx[j + 1], P = D.ra[j], Q = D.ra[j + 1];
@@ -702,26 +702,33 @@ __device__ double gang_build_right(GangCtx& C, int i, bool* ok) {
 // and multiplies its own rows by the inverse (one GEMM); the first pass
 // shifts the Gram matrix by 11 (m c + c (c + 1)) u ||W||_F^2 so that it stays
 // positive definite for condition numbers up to ~1/u.  The c x c work runs in
-// LDS when 2 c^2 + c doubles fit after the GEMM tiles, else in the member's
-// global slots.  The panel is copied from g: forward W[row, col] =
+// LDS: by waves (cholqr_wave_step) for c <= 64 where 3 c^2 + 128 doubles fit
+// after the GEMM tiles, else by the whole workgroup where 2 c^2 + c fit, else
+// in the member's global slots.  The panel is copied from g: forward W[row, col] =
 // g[row c + col] (m = a n, c = b), backward W[row, col] = g[col m + row]
 // (m = n b, c = a).  On success *Q is the panel's Q (own rows valid, row
 // stride c, in D.qw or D.qq) and *R the upper c x c factor; returns 0, or 1
 // when a pivot failed (every member alike), 2 non-finite, -1 aborted.
-__device__ int gang_cholqr(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl,
+__device__ TT_COLD int gang_cholqr(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl,
                            const double** Qout, const double** Rout) {
   const GangDesc& D = C.D;
   int m0, m1;
   gang_span(m, C.G, C.g, m0, m1);
   const int rows = m1 - m0;
   const long cc = (long)c * c;
-  double *Rp, *Rt, *tmp;
-  if (GEMM_LDS_DOUBLES + 2 * cc + c <= C.lds_cap) {
+  double *Rp, *Rt, *tmp, *Rinv;
+  const bool small = c <= 64 && GEMM_LDS_DOUBLES + 3 * cc + 128 <= C.lds_cap;
+  if (small) {
     Rp = C.lds + GEMM_LDS_DOUBLES;
+    Rt = Rp + cc;
+    Rinv = Rt + cc;
+    tmp = Rinv + cc;
+  } else if (GEMM_LDS_DOUBLES + 2 * cc + c <= C.lds_cap) {
+    Rp = Rinv = C.lds + GEMM_LDS_DOUBLES;
     Rt = Rp + cc;
     tmp = Rt + cc;
   } else {
-    Rp = D.qrs + (long)C.g * 3 * D.rmax2;
+    Rp = Rinv = D.qrs + (long)C.g * 3 * D.rmax2;
     Rt = Rp + D.rmax2;
     tmp = Rt + D.rmax2;
   }
@@ -765,10 +772,10 @@ __device__ int gang_cholqr(GangCtx& C, const double* g, int m, int c, bool trans
       __syncthreads();
     }
     // Cholesky, R accumulation and the inverse factor (identical in every member)
-    if (!cholqr_small_step(Rp, Rt, tmp, c)) return 1;
+    if (!(small ? cholqr_wave_step(Rp, Rt, Rinv, tmp, c) : cholqr_small_step(Rp, Rt, tmp, c))) return 1;
     // own rows: W <- W R^{-1}
     if (rows > 0)
-      wg_gemm<double, double>(rows, c, c, crm<double>(Win + (long)m0 * c, c), crm<double>(Rp, c),
+      wg_gemm<double, double>(rows, c, c, crm<double>(Win + (long)m0 * c, c), crm<double>(Rinv, c),
                               mrm<double>(Wout + (long)m0 * c, c), C.lds);
     __syncthreads();
     double* t = Win;
@@ -814,7 +821,7 @@ __device__ void rows_dots(const double* V, const double* X, int c, int j, int r_
 // formed by applying the reflectors to [I; 0] backwards (one reduction per
 // column).  Rows as in gang_cholqr; *Q in D.qq (own rows), *R in D.rf.
 // Returns 0, or -1 when the gang aborted.
-__device__ int gang_hhqr(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl, const double** Qout,
+__device__ TT_COLD int gang_hhqr(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl, const double** Qout,
                          const double** Rout) {
   const GangDesc& D = C.D;
   SolveLDS& S = C.S;
@@ -1007,7 +1014,7 @@ __device__ int gang_hhqr_run(GangCtx& C, int m, int c) {
   return 0;
 }
 
-__device__ int gang_hhqr_blocked(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl,
+__device__ TT_COLD int gang_hhqr_blocked(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl,
                                  const double** Qout, const double** Rout) {
   const GangDesc& D = C.D;
   int m0, m1;
@@ -1036,7 +1043,7 @@ __device__ int gang_hhqr_blocked(GangCtx& C, const double* g, int m, int c, bool
 // reference's QR does) or, for a rank-deficient panel too tall for that, the
 // split column sweep.  After one failed pivot the system skips the Cholesky
 // QR.  Returns false once the gang has aborted.
-__device__ bool gang_ortho_right(GangCtx& C, double* fl) {
+__device__ TT_COLD bool gang_ortho_right(GangCtx& C, double* fl) {
   const GangDesc& D = C.D;
   SolveLDS& S = C.S;
   for (int i = D.d - 1; i >= 1; --i) {

@@ -6,8 +6,8 @@
 // two resident workgroups per CU.  With registers to spare, the blocked
 // QR's streaming passes keep eight rows per lane in flight and the global
 // GEMMs two K-steps (same arithmetic order as k_als's two rows and one step).
-#define TTALS_HH_ROWS 8
-#define TTALS_GEMM_PREFETCH 2
+#define TTALS_NT 512
+#define TTALS_HH_ROWS 4
 #include "ttals_hybrid.hpp"
 
 namespace ttals {
@@ -39,6 +39,8 @@ hipError_t hybrid_static_lds(size_t* bytes) {
   if (e == hipSuccess) *bytes = fa.sharedSizeBytes;
   return e;
 }
+
+long hybrid_min_arena() { return GEMM_LDS_DOUBLES; }
 
 hipError_t hybrid_launch(int blocks, size_t dyn_lds, hipStream_t stream, const GangDesc* gdescs,
                          const int* block_sys, int gang_blocks, const SysDesc* descs, long arena) {

@@ -13,6 +13,9 @@ hipError_t hybrid_occupancy(int* per_cu, size_t dyn_lds);
 // Static LDS bytes of k_hybrid.
 hipError_t hybrid_static_lds(size_t* bytes);
 
+// Smallest arena (doubles) its GEMM staging tiles need.
+long hybrid_min_arena();
+
 // Launches k_hybrid: `blocks` workgroups, the first `gang_blocks` of them the
 // gangs of `gdescs` (block_sys: gang of each), the rest one system each of
 // `descs`, in order.
