@@ -833,6 +833,8 @@ struct ttals_ctx {
   size_t hst_bytes = 0;
   hipEvent_t done = nullptr;  // completion of the last submission
   hipEvent_t k0 = nullptr, k1 = nullptr;  // bracket the last k_als launch (timing events)
+  hipStream_t side = nullptr;             // runs the small systems of a batch beside its large ones
+  hipEvent_t fork = nullptr, join = nullptr;
   bool timed = false;
   bool inflight = false;
   std::vector<Pending> pending;
@@ -1228,9 +1230,29 @@ struct Placement {
   size_t dev_cap;
 };
 
-// Plans and enqueues one k_als launch for a batch (descriptors, one metadata
-// copy, the launch, the result copy).  On return *r_res is the staging offset
-// of the compact results (res_stride doubles per system).
+int hybrid_arena(ttals_ctx* c, long* out);
+
+// Does a single-workgroup sle system take the wide kernel (k_hybrid: eight
+// waves, one system per CU) instead of k_als (four waves, two per CU)?  A rule
+// on the system alone, so that its result does not depend on the batch it
+// comes in.  Eight waves shorten a system that works from global memory (alone
+// on the device, 12 cores: n = 16, rank 16 / 24 / 32: 8.6 / 19.1 / 29.2 ms on
+// k_als, 7.4 / 14.7 / 21.3 ms here), but hold half as many: 512 equal systems
+// take 16.0 / 39.4 / 71.4 ms on k_als and 18.1 / 40.4 / 68.5 ms here.  The line
+// lies where a full device does not lose (n = 8, rank 32, N = 8192: 30.6 and
+// 32.4 ms; rank 48, N = 18432: 84.3 and 80.3 ms); an uneven batch, which lasts
+// as long as its largest systems, gains below it too.
+constexpr long WIDE_FROM = 10240;  // unknowns of the largest local problem
+bool wide_system(const ttals_tt& A, const ttals_tt& x0) {
+  for (int i = 0; i < A.order; ++i)
+    if ((long)x0.ranks[i] * A.row_dims[i] * x0.ranks[i + 1] >= WIDE_FROM) return true;
+  return false;
+}
+
+// Plans and enqueues one batch (descriptors, one metadata copy, the launch --
+// two side by side for an sle batch of wide and small systems -- and the
+// result copy).  On return *r_res is the staging offset of the compact results
+// (res_stride doubles per system).
 int enqueue_batch(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, Placement& pl, size_t* r_res,
                   size_t* res_stride_out, bool timed) {
   const int kind = B.kind, count = B.count;
@@ -1246,11 +1268,19 @@ int enqueue_batch(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, Placemen
   int dmax = 0;
   SysSizes z;
   SysOff o;
+  const long arena = std::max<long>(c->arena, GEMM_LDS_DOUBLES);
+  // wide systems (an arena the caller chose keeps everything on k_als)
+  std::vector<char> wide(count, 0);
+  int nwide = 0;
   for (int s = 0; s < count; ++s) {
     int rc = size_system(c, kind, B.A[s], B.x0[s], kind == 0 ? &B.b[s] : nullptr, B.xo[s], s, z);
     if (rc) return rc;
     take_offsets(kind, z, hl, dl, o);
     dmax = std::max(dmax, z.d);
+    if (kind == 0 && !c->arena_set && wide_system(B.A[s], B.x0[s])) {
+      wide[s] = 1;
+      ++nwide;
+    }
   }
   const size_t meta_bytes = hl.bytes;
   // compact results: one row of 16 scalars + (dmax+1) ranks per system, on
@@ -1279,24 +1309,45 @@ int enqueue_batch(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, Placemen
   auto dptr = [&](size_t off) { return reinterpret_cast<void*>(dmeta + off); };
   auto wptr = [&](size_t off) { return reinterpret_cast<double*>(dbase + off); };
   SysDesc* hdesc = reinterpret_cast<SysDesc*>(hbase + m_descs);
-  // pass 2: the same offsets again, descriptors written
+  // pass 2: the same offsets again, descriptors written (wide systems first)
   Layout hl2, dl2;
   (void)hl2.take(sizeof(SysDesc) * count);
+  int at_wide = 0, at_small = nwide;
   for (int s = 0; s < count; ++s) {
     (void)size_system(c, kind, B.A[s], B.x0[s], kind == 0 ? &B.b[s] : nullptr, B.xo[s], s, z);
     take_offsets(kind, z, hl2, dl2, o);
-    fill_sys(c, B, s, o, hbase, dmeta, dbase, reinterpret_cast<double*>(dbase + w_res) + res_stride * s, hdesc[s]);
+    fill_sys(c, B, s, o, hbase, dmeta, dbase, reinterpret_cast<double*>(dbase + w_res) + res_stride * s,
+             hdesc[wide[s] ? at_wide++ : at_small++]);
   }
   HIPCHK(c, hipMemcpyAsync(dmeta, hbase, meta_bytes, hipMemcpyHostToDevice, stream));
-  const long arena = std::max<long>(c->arena, GEMM_LDS_DOUBLES);
   if (timed) {
     if (!c->k0) HIPCHK(c, hipEventCreate(&c->k0));
     if (!c->k1) HIPCHK(c, hipEventCreate(&c->k1));
     HIPCHK(c, hipEventRecord(c->k0, stream));
   }
-  hipLaunchKernelGGL(kind == 0 ? k_als<0> : k_als<1>, dim3(count), dim3(NT), (size_t)arena * 8, stream,
-                     (const SysDesc*)dptr(m_descs), arena);
-  HIPCHK(c, hipGetLastError());
+  const SysDesc* ddesc = (const SysDesc*)dptr(m_descs);
+  const int nsmall = count - nwide;
+  // both classes: the small systems on the side stream, after the wide launch
+  // has taken its CUs; the caller's stream goes on when both are done
+  const bool both = nwide > 0 && nsmall > 0;
+  if (both) HIPCHK(c, hipEventRecord(c->fork, stream));
+  if (nwide > 0) {
+    long harena = 0;
+    int rc;
+    if ((rc = hybrid_arena(c, &harena))) return rc;
+    HIPCHK(c, hybrid_launch(nwide, (size_t)harena * 8, stream, nullptr, nullptr, 0, ddesc, harena));
+  }
+  if (nsmall > 0) {
+    hipStream_t st = both ? c->side : stream;
+    if (both) HIPCHK(c, hipStreamWaitEvent(st, c->fork, 0));
+    hipLaunchKernelGGL(kind == 0 ? k_als<0> : k_als<1>, dim3(nsmall), dim3(NT), (size_t)arena * 8, st, ddesc + nwide,
+                       arena);
+    HIPCHK(c, hipGetLastError());
+    if (both) {
+      HIPCHK(c, hipEventRecord(c->join, st));
+      HIPCHK(c, hipStreamWaitEvent(stream, c->join, 0));
+    }
+  }
   if (timed) {
     HIPCHK(c, hipEventRecord(c->k1, stream));
     c->timed = true;
@@ -1943,6 +1994,17 @@ int ttals_ctx_create(int device, ttals_ctx** out) {
     const long kb = std::atol(e);
     if (kb >= 0 && kb <= 61) c->arena = kb * 1024 / 8;
   }
+  // the side stream and its events, here once (the allocation-free entry point creates nothing)
+  int prev = 0;
+  bool ok = hipGetDevice(&prev) == hipSuccess && hipSetDevice(device) == hipSuccess;
+  ok = ok && hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) == hipSuccess;
+  ok = ok && hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) == hipSuccess;
+  ok = ok && hipEventCreateWithFlags(&c->join, hipEventDisableTiming) == hipSuccess;
+  (void)hipSetDevice(prev);
+  if (!ok) {
+    ttals_ctx_destroy(c);
+    return TTALS_E_HIP;
+  }
   *out = c;
   return 0;
 }
@@ -1956,6 +2018,9 @@ void ttals_ctx_destroy(ttals_ctx* c) {
   }
   if (c->k0) (void)hipEventDestroy(c->k0);
   if (c->k1) (void)hipEventDestroy(c->k1);
+  if (c->fork) (void)hipEventDestroy(c->fork);
+  if (c->join) (void)hipEventDestroy(c->join);
+  if (c->side) (void)hipStreamDestroy(c->side);
   if (c->dws) (void)hipFree(c->dws);
   if (c->hst) (void)hipHostFree(c->hst);
   delete c;

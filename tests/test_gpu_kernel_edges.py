@@ -166,3 +166,28 @@ def test_local_lu(lib, a, P, n, Q, b, kb):
         assert lib.ttals_set_arena_kb(ctx, 61) == 0
     res = float((M @ v - f).norm())
     assert res <= 4 * N * N * EPS * float(M.norm()) * float(v.norm())
+
+
+def test_one_schedule_result_does_not_depend_on_the_batch(lib):
+    """Systems on both sides of the line between the two single-workgroup
+    kernels (10240 unknowns): in one batch, in another order and alone, the
+    same bits."""
+    from scikit_tt_amd import tensor_train as tt, workloads as W
+    from scikit_tt_amd.solvers import sle
+    rng = np.random.default_rng(3)
+    sizes = [(4, 16, 25), (4, 4, 4), (4, 16, 26), (5, 3, 7), (4, 41, 16)]  # N: 10000, 64, 10816, 147, 10496
+    A = tt.from_host_batch([W.shifted_operator(rng, d, n) for d, n, r in sizes])
+    b = tt.from_host_batch([W.random_tt(rng, [n] * d, 3) for d, n, r in sizes])
+    x = tt.from_host_batch([W.random_tt(rng, [n] * d, [1] + [r] * (d - 1) + [1]) for d, n, r in sizes])
+    together = sle.als_batch(A, x, b)
+    back = sle.als_batch(A[::-1], x[::-1], b[::-1])
+    for s in range(len(sizes)):
+        alone = sle.als_batch(A[s:s + 1], x[s:s + 1], b[s:s + 1])[0]
+        for t in (together[s], back[len(sizes) - 1 - s]):
+            assert t.ranks == alone.ranks
+            for c1, c2 in zip(t.device_cores, alone.device_cores):
+                assert torch.equal(c1, c2)
+        full = alone.matricize()
+        want = A[s].dot(alone).matricize()
+        assert np.linalg.norm(want - b[s].matricize()) <= 0.5 * np.linalg.norm(b[s].matricize())
+        assert np.isfinite(full).all()
