@@ -21,6 +21,16 @@ constexpr int NT = TTALS_NT;
 constexpr int NWAVE = NT / 64;
 static_assert(NT == 256 || NT == 512, "the tile shapes below assume 4 or 8 waves");
 
+// Arguments of out-of-line functions arrive in vector registers: back to
+// scalars, so that bounds are uniform branches and bases scalar addresses.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <class T>
+__device__ __forceinline__ T* uni(T* p) {
+  const unsigned long v = reinterpret_cast<unsigned long>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+  return reinterpret_cast<T*>(((unsigned long)hi << 32) | lo);
+}
+
 // f(0), ..., f(N - 1) with the index a compile-time constant (register arrays)
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -737,15 +747,17 @@ __device__ __forceinline__ void wg_copy_opcore_pnmq(const double* src, double* d
 // partial sums meet in `red` in a fixed order.  Operands are loaded four
 // K-steps ahead of their MFMAs; indices past M, N or K read a clamped
 // in-range address and contribute zero.
-__device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int acs, const double* B_, int brs,
-                            int bcs, double* C_, const FMap& cr, const FMap& cc, double* red_, int red_cap) {
+template <class T>
+__device__ void mf_gemm_lin(int M, int N, int K, const T* A_, int ars, int acs, const T* B_, int brs, int bcs, T* C_,
+                            const FMap& cr, const FMap& cc, T* red_, int red_cap) {
+  typedef typename std::conditional<std::is_same<T, double>::value, dx4_t, fx4_t>::type acc_t;
   M = __builtin_amdgcn_readfirstlane(M);
   N = __builtin_amdgcn_readfirstlane(N);
   K = __builtin_amdgcn_readfirstlane(K);
-  const TT_LDS double* pa = (const TT_LDS double*)A_;
-  const TT_LDS double* pb = (const TT_LDS double*)B_;
-  TT_LDS double* pc = (TT_LDS double*)C_;
-  TT_LDS double* red = (TT_LDS double*)red_;
+  const TT_LDS T* pa = (const TT_LDS T*)A_;
+  const TT_LDS T* pb = (const TT_LDS T*)B_;
+  TT_LDS T* pc = (TT_LDS T*)C_;
+  TT_LDS T* red = (TT_LDS T*)red_;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lk = lane >> 4;
@@ -773,7 +785,7 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
     for (int u = w; u < tiles; u += 2 * NWAVE) {
       const bool two = u + NWAVE < tiles;
       const int tt[2] = {u, two ? u + NWAVE : u};
-      const TT_LDS double *ap[2], *bp[2], *alast[2], *blast[2];
+      const TT_LDS T *ap[2], *bp[2], *alast[2], *blast[2];
       int ti[2], jj[2];
       bool jv[2];
 #pragma unroll
@@ -791,10 +803,10 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
         bp[h] += __mul24(lk, brs);
       }
       int k = lk;
-      dx4_t acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+      acc_t acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
       int s = 0;
       for (; s + 4 <= ks; s += 4) {
-        double av[2][4], bv[2][4];
+        T av[2][4], bv[2][4];
         bool kv[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -813,15 +825,15 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
         for (int q = 0; q < 4; ++q)
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[h][q], kv[q] ? bv[h][q] : 0.0, acc[h], 0, 0, 0);
+            acc[h] = mfma16x16x4(av[h][q], kv[q] ? bv[h][q] : (T)0, acc[h]);
       }
       for (; s < ks; ++s) {
         const bool kq = k < K;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const double x = (kq ? ap[h] : alast[h])[0];
-          const double y = (kq ? bp[h] : blast[h])[0];
-          acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, kq ? y : 0.0, acc[h], 0, 0, 0);
+          const T x = (kq ? ap[h] : alast[h])[0];
+          const T y = (kq ? bp[h] : blast[h])[0];
+          acc[h] = mfma16x16x4(x, kq ? y : (T)0, acc[h]);
           ap[h] += acs4;
           bp[h] += brs4;
         }
@@ -834,7 +846,7 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
           const int cj = fmap_at(cc, jj[h]);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int row = (ti[h] << 4) + lk + 4 * e;
+            const int row = (ti[h] << 4) + mfma16_row<T>(lk, e);
             if (row < M) pc[fmap_at(cr, row) + cj] = acc[h][e];
           }
         }
@@ -855,17 +867,17 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
     // columns past N read a clamped address: their outputs are discarded.  A
     // K index past the end reads the last column/row instead and its B value
     // is zeroed (A finite there, so the product vanishes).
-    const TT_LDS double* ap = pa + __mul24(iv ? i : M - 1, ars);
-    const TT_LDS double* bp = pb + __mul24(jv ? j : N - 1, bcs);
-    const TT_LDS double* alast = ap + __mul24(K - 1, acs);
-    const TT_LDS double* blast = bp + __mul24(K - 1, brs);
+    const TT_LDS T* ap = pa + __mul24(iv ? i : M - 1, ars);
+    const TT_LDS T* bp = pb + __mul24(jv ? j : N - 1, bcs);
+    const TT_LDS T* alast = ap + __mul24(K - 1, acs);
+    const TT_LDS T* blast = bp + __mul24(K - 1, brs);
     ap += __mul24((s0 << 2) + lk, acs);
     bp += __mul24((s0 << 2) + lk, brs);
     int k = (s0 << 2) + lk;
-    dx4_t acc = {0.0, 0.0, 0.0, 0.0};
+    acc_t acc = {0, 0, 0, 0};
     int s = s0;
     for (; s + 4 <= s1; s += 4) {
-      double av[4], bv[4];
+      T av[4], bv[4];
       bool kv[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -880,13 +892,13 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], kv[q] ? bv[q] : 0.0, acc, 0, 0, 0);
+        acc = mfma16x16x4(av[q], kv[q] ? bv[q] : (T)0, acc);
     }
     for (; s < s1; ++s) {
       const bool kq = k < K;
-      const double x = (kq ? ap : alast)[0];
-      const double y = (kq ? bp : blast)[0];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, kq ? y : 0.0, acc, 0, 0, 0);
+      const T x = (kq ? ap : alast)[0];
+      const T y = (kq ? bp : blast)[0];
+      acc = mfma16x16x4(x, kq ? y : (T)0, acc);
       ap += acs4;
       bp += brs4;
       k += 4;
@@ -894,14 +906,14 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
     if (groups > 1) {
       // one work item per wave: partial parts park their sums, part 0 adds them
       if (part > 0) {
-        TT_LDS double* r = red + ((part - 1) * tiles + t) * 256 + lane * 4;
+        TT_LDS T* r = red + ((part - 1) * tiles + t) * 256 + lane * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] = acc[e];
       }
       __syncthreads();
       if (part > 0) break;
       for (int p2 = 1; p2 < groups; ++p2) {
-        const TT_LDS double* r = red + ((p2 - 1) * tiles + t) * 256 + lane * 4;
+        const TT_LDS T* r = red + ((p2 - 1) * tiles + t) * 256 + lane * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] += r[e];
       }
@@ -910,7 +922,7 @@ __device__ void mf_gemm_lin(int M, int N, int K, const double* A_, int ars, int 
       const int cj = fmap_at(cc, j);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int row = (ti << 4) + lk + 4 * e;
+        const int row = (ti << 4) + mfma16_row<T>(lk, e);
         if (row < M) pc[fmap_at(cr, row) + cj] = acc[e];
       }
     }
@@ -960,12 +972,12 @@ __device__ __attribute__((noinline)) void local_matvec_mf(int a, int P, int n, i
   const int s1 = odd_stride(P * n), s2 = odd_stride(b * Q);
   const FMap plain_r = fmap(1, b, 0), plain_c = fmap(1, 1, 0);
   // T1[(P,a'), (n,b)]: A = L viewed (P*a, a) with rows contiguous, B = v (a, n*b)
-  mf_gemm_lin(P * a, n * b, a, L, 1, P * a, v, n * b, 1, t1, pl.c1r, pl.c1c, nullptr, 0);
+  mf_gemm_lin(P * a, n * b, a, L, 1, P * a, v, n * b, 1, t1, pl.c1r, pl.c1c, (double*)nullptr, 0);
   // T2[(a',b), (m,Q)]: A = T1 rows (stride s1), B = A' (P*n, n*Q)
   if (P * n <= 16 && P * n * n * Q <= 64)
     stage2_valu(a, P, n, Q, b, t1, Ap, t2);
   else
-    mf_gemm_lin(a * b, n * Q, P * n, t1, s1, 1, Ap, n * Q, 1, t2, pl.c2r, pl.c2c, nullptr, 0);
+    mf_gemm_lin(a * b, n * Q, P * n, t1, s1, 1, Ap, n * Q, 1, t2, pl.c2r, pl.c2c, (double*)nullptr, 0);
   // y[(a',m), b']: A = T2 rows (stride s2), B = R (b*Q, b); T1 is free: K-split scratch
   mf_gemm_lin(a * n, b, b * Q, t2, s2, 1, R, b, 1, y, plain_r, plain_c, t1, (int)ds_t1_size(a, P, n, b));
 }
@@ -982,12 +994,12 @@ __device__ __attribute__((noinline)) void stack_left_mf(int a, int P, int n, int
                                                         double* t2) {
   const MvPlan pl = mv_plan(a, P, n, Q, b);
   const int s1 = odd_stride(P * n), s2 = odd_stride(b * Q);
-  mf_gemm_lin(P * a, n * b, a, L, 1, P * a, x, n * b, 1, t1, pl.c1r, pl.c1c, nullptr, 0);
+  mf_gemm_lin(P * a, n * b, a, L, 1, P * a, x, n * b, 1, t1, pl.c1r, pl.c1c, (double*)nullptr, 0);
   if (P * n <= 16 && P * n * n * Q <= 64)
     stage2_valu(a, P, n, Q, b, t1, Ap, t2);
   else
-    mf_gemm_lin(a * b, n * Q, P * n, t1, s1, 1, Ap, n * Q, 1, t2, pl.c2r, pl.c2c, nullptr, 0);
-  mf_gemm_lin(b * Q, b, a * n, t2, 1, s2, x, b, 1, out, fmap(1, b, 0), fmap(1, 1, 0), nullptr, 0);
+    mf_gemm_lin(a * b, n * Q, P * n, t1, s1, 1, Ap, n * Q, 1, t2, pl.c2r, pl.c2c, (double*)nullptr, 0);
+  mf_gemm_lin(b * Q, b, a * n, t2, 1, s2, x, b, 1, out, fmap(1, b, 0), fmap(1, 1, 0), (double*)nullptr, 0);
 }
 
 // The operator core (P, m, n, Q) copied into LDS as A'(Q, n, m, P): the
@@ -1065,7 +1077,7 @@ __device__ __attribute__((noinline)) void local_matvec_m2(int a, int P, int n, i
                                                           double* red) {
   const int nb = n * b, k2 = P * n * b, s = odd_stride(k2);
   const FMap plain = fmap(1, 1, 0);
-  mf_gemm_lin(P * a, nb, a, L, 1, P * a, v, nb, 1, t1, fmap(a, nb, s), plain, nullptr, 0);
+  mf_gemm_lin(P * a, nb, a, L, 1, P * a, v, nb, 1, t1, fmap(a, nb, s), plain, (double*)nullptr, 0);
   mf_gemm_lin(a, nb, k2, t1, s, 1, M2, nb, 1, y, fmap(1, nb, 0), plain, red, m2_red_need(a, nb));
 }
 

@@ -305,6 +305,9 @@ struct GangCtx {
   // set once a Cholesky QR of this system failed (a numerically
   // rank-deficient panel): its later panels go to Householder directly
   bool chol_off = false;
+  // bytes per element of the operator pieces held in LDS for the Krylov
+  // iterations of the current local problem (gang_op_lds; 0: none)
+  int op_lds = 0;
   __device__ bool sync() {
     const long long t0 = ph_now();
     const bool r = gang_sync(D.sync, G);
@@ -359,6 +362,123 @@ __device__ __forceinline__ GangLocal gang_local(const GangCtx& C, int i) {
   return o;
 }
 
+// LDS of the on-chip matvec of a member with s rows a' (elements of T, after
+// the GEMM staging tiles, which the reductions use): L's rows, the operator
+// core as A'(P, n, m, Q), R, the two intermediates (the first also the result).
+template <class T>
+struct GangOpLDS {
+  T *L, *A, *R, *t1, *t2;
+  __device__ GangOpLDS(double* lds, int a, int P, int n, int Q, int b, int s) {
+    L = reinterpret_cast<T*>(lds + GEMM_LDS_DOUBLES);
+    A = L + (long)a * P * s;
+    R = A + (long)P * n * n * Q;
+    t1 = R + (long)b * Q * b;
+    t2 = t1 + t1_size(s, P, n, b);
+  }
+  static __device__ long t1_size(int s, int P, int n, int b) {
+    const long t1 = ds_t1_size(s, P, n, b), y = (long)s * n * b;
+    return t1 > y ? t1 : y;
+  }
+  static __device__ bool fits(long cap, int a, int P, int n, int Q, int b, int s) {
+    const long e = (long)a * P * s + (long)P * n * n * Q + (long)b * Q * b + t1_size(s, P, n, b) + ds_t2_size(s, n, Q, b);
+    return P * s <= SKINNY_M && 8 * (cap - GEMM_LDS_DOUBLES) >= (long)sizeof(T) * e;
+  }
+};
+
+// Puts the member's operator pieces into LDS for the Krylov iterations of one
+// local problem, where they fit and its rows are few (P s <= SKINNY_M: the
+// first stage keeps one accumulator per row and output column).
+template <class T>
+__device__ TT_COLD void gang_op_lds(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R) {
+  const int s = o.r1 - o.r0;
+  C.op_lds = 0;
+  if (s > 0 && GangOpLDS<T>::fits(C.lds_cap, o.a, o.P, o.n, o.Q, o.b, s)) {
+    const GangOpLDS<T> S(C.lds, o.a, o.P, o.n, o.Q, o.b, s);
+    const int ps = o.P * s;
+    for (int e = threadIdx.x; e < o.a * ps; e += NT) {
+      const int k = e / ps, i = e - k * ps, p = i / s;
+      S.L[e] = L[((long)k * o.P + p) * o.a + o.r0 + (i - p * s)];
+    }
+    const int tot = o.P * o.n * o.n * o.Q;
+    const float iQ = 1.0f / (float)o.Q, in = 1.0f / (float)o.n;
+    for (int e = threadIdx.x; e < tot; e += NT) {  // (P, m, n, Q) -> (P, n, m, Q)
+      const int r1 = fquot(e, iQ), q = e - r1 * o.Q;
+      const int r2 = fquot(r1, in), nn = r1 - r2 * o.n;
+      const int p = fquot(r2, in), mm = r2 - p * o.n;
+      S.A[((p * o.n + nn) * o.n + mm) * o.Q + q] = A[e];
+    }
+    for (int e = threadIdx.x; e < o.b * o.Q * o.b; e += NT) S.R[e] = R[e];
+    C.op_lds = (int)sizeof(T);
+  }
+  __syncthreads();
+}
+
+// The member's rows of y = M v with the operator and both intermediates in
+// LDS.  v is read whole (it is complete in global memory), each element once;
+// the contractions after that see no global latency.  The global form
+// (gang_matvec) writes and reads both intermediates through L2 and pays a
+// round trip per K-step of each GEMM: 37.7 ms against 18.9 ms for two sweeps
+// of a system of order 4, n = 32, ranks 32, on 32 members (412 iterations).
+template <class T>
+__device__ TT_COLD void gang_matvec_lds(const GangCtx& C, const GangLocal& o_, const T* v, T* y) {
+  const int a = uni(o_.a), P = uni(o_.P), n = uni(o_.n), Q = uni(o_.Q), b = uni(o_.b), r0 = uni(o_.r0), s = uni(o_.r1) - r0;
+  const GangOpLDS<T> S(C.lds, a, P, n, Q, b, s);
+  const int ps = P * s, nb = n * b, s1 = odd_stride(P * n), s2 = odd_stride(b * Q);
+  const TT_LDS T* Ls = (const TT_LDS T*)S.L;
+  TT_LDS T* t1 = (TT_LDS T*)S.t1;
+  const float ib = 1.0f / (float)b, is = 1.0f / (float)s;
+  // T1[(a'_l, b), (P, n)] = sum_a L[a, P, r0 + a'_l] v[a, n, b]: a thread per
+  // column (n, b), eight loads of v in flight
+  for (int j = threadIdx.x; j < nb; j += NT) {
+    T acc[SKINNY_M];
+#pragma unroll
+    for (int i = 0; i < SKINNY_M; ++i) acc[i] = (T)0;
+    const T* vp = v + j;
+    int k = 0;
+    for (; k + 8 <= a; k += 8) {
+      T x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = vp[(long)(k + u) * nb];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int i = 0; i < SKINNY_M; ++i)
+          if (i < ps) acc[i] += Ls[(k + u) * ps + i] * x[u];
+    }
+    for (; k < a; ++k) {
+      const T x = vp[(long)k * nb];
+#pragma unroll
+      for (int i = 0; i < SKINNY_M; ++i)
+        if (i < ps) acc[i] += Ls[k * ps + i] * x;
+    }
+    const int nn = fquot(j, ib), bb = j - nn * b;
+#pragma unroll
+    for (int i = 0; i < SKINNY_M; ++i)
+      if (i < ps) {
+        const int p = fquot(i, is), al = i - p * s;
+        t1[(al * b + bb) * s1 + p * n + nn] = acc[i];
+      }
+  }
+  __syncthreads();
+  // T2[(a'_l, m), (b, Q)] and y[(a'_l, m), b'] as on-chip matrix-core GEMMs
+  mf_gemm_lin<T>(s * b, n * Q, P * n, S.t1, s1, 1, S.A, n * Q, 1, S.t2, fmap(b, n * s2, Q), fmap(Q, s2, 1), (T*)nullptr,
+                 0);
+  mf_gemm_lin<T>(s * n, b, b * Q, S.t2, s2, 1, S.R, b, 1, S.t1, fmap(1, b, 0), fmap(1, 1, 0), (T*)nullptr, 0);
+  T* yo = y + (long)r0 * nb;
+  for (int e = threadIdx.x; e < s * nb; e += NT) yo[e] = t1[e];
+  __syncthreads();
+}
+
+template <class T>
+__device__ __forceinline__ void gang_apply(const GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R,
+                                           const T* v, T* y) {
+  if (C.op_lds == (int)sizeof(T))
+    gang_matvec_lds<T>(C, o, v, y);
+  else
+    gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, v, y, o.r0, o.r1, reinterpret_cast<T*>(C.t1),
+                   reinterpret_cast<T*>(C.t2), reinterpret_cast<T*>(C.lds));
+}
+
 // Conjugate gradients on M x = f (x holds the start), vectors of type T,
 // matvec on operands (L, A, R) of type T, reductions in FP64.  Returns 0
 // converged, 1 p^T M p <= 0 (not SPD), 2 maxit, -1 gang aborted.
@@ -368,11 +488,8 @@ __device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const
   const int G = C.G, g = C.g;
   const int ld = GANG_LD;
   double* part = C.D.part;
-  T* t1 = reinterpret_cast<T*>(C.t1);
-  T* t2 = reinterpret_cast<T*>(C.t2);
-  T* lds = reinterpret_cast<T*>(C.lds);
   // r = f - M x, p = r; |f|, |r|
-  gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, x, q, o.r0, o.r1, t1, t2, lds);
+  gang_apply<T>(C, o, L, A, R, x, q);
   double ff = 0.0, rr = 0.0;
   for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) {
     const double fe = (double)f[e], re = fe - (double)q[e];
@@ -398,7 +515,7 @@ __device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const
   while (*iters < maxit) {
     // q = M p (p complete: the barrier above / at the end of the last step)
     const long long tm = ph_now();
-    gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, p, q, o.r0, o.r1, t1, t2, lds);
+    gang_apply<T>(C, o, L, A, R, p, q);
     ph_add(C.S, PH_MATVEC, tm);
     double pq = 0.0;
     for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) pq += (double)p[e] * (double)q[e];
@@ -446,9 +563,6 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
   const int ld = GANG_LD;
   double* part = C.D.part;
   SolveLDS& S = C.S;
-  T* t1 = reinterpret_cast<T*>(C.t1);
-  T* t2 = reinterpret_cast<T*>(C.t2);
-  T* lds = reinterpret_cast<T*>(C.lds);
   const long N = o.N;
   if (m > KMAX) m = KMAX;
   if (m > o.N) m = o.N;
@@ -467,7 +581,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
   }
   for (;;) {
     // w = f - M x; beta = |w|; v_0 = w / beta
-    gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, x, w, o.r0, o.r1, t1, t2, lds);
+    gang_apply<T>(C, o, L, A, R, x, w);
     double bb = 0.0;
     for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) {
       const double we = (double)f[e] - (double)w[e];
@@ -494,7 +608,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
     bool brk = false;
     for (int j = 0; j < m; ++j) {
       const long long tm = ph_now();
-      gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, V + (long)j * N, w, o.r0, o.r1, t1, t2, lds);
+      gang_apply<T>(C, o, L, A, R, V + (long)j * N, w);
       ph_add(S, PH_MATVEC, tm);
       double* col = S.H + j * (KMAX + 1);  // column j (rows 0..j+1), identical in every member
       for (int k = threadIdx.x; k <= j + 1; k += NT) col[k] = 0.0;
@@ -583,7 +697,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
     }
     if (*iters >= maxit) {
       // final residual decides
-      gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, x, w, o.r0, o.r1, t1, t2, lds);
+      gang_apply<T>(C, o, L, A, R, x, w);
       double tr = 0.0;
       for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) {
         const double we = (double)f[e] - (double)w[e];
@@ -1140,6 +1254,7 @@ __device__ int gang_step(GangCtx& C, int i, bool forward, bool sym, StepStats& s
   double vfl = 0.0;
   if (D.prec == 0) {
     r = 1;
+    gang_op_lds<double>(C, o, o.L, o.A, o.R);
     if (sym) r = gang_cg<double>(C, o, o.L, o.A, o.R, D.g, D.f, D.r, D.p, D.q, D.tol, D.maxit, &its, &vfl);
     if (r == 1) r = gang_gmres<double>(C, o, o.L, o.A, o.R, D.g, D.f, D.q, D.V, D.tol, D.maxit, D.gm_restart, &its,
                                         &vfl, &unconf);
@@ -1158,6 +1273,7 @@ __device__ int gang_step(GangCtx& C, int i, bool forward, bool sym, StepStats& s
       }
     }
     if (!C.sync()) return ST_ABORT;
+    gang_op_lds<float>(C, o, D.L32, D.A32, D.R32);
     r = 2;
     int inner_total = 0;
     for (int outer = 0; outer < 30; ++outer) {

@@ -87,16 +87,6 @@ __device__ __forceinline__ double rows4_sum(double v) {
   return __hiloint2double(b.x, a.x) + __hiloint2double(b.y, a.y);
 }
 
-// Arguments of out-of-line functions arrive in vector registers: back to
-// scalars, so that bounds are uniform branches and bases scalar addresses.
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-template <class T>
-__device__ __forceinline__ T* uni(T* p) {
-  const unsigned long v = reinterpret_cast<unsigned long>(p);
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-  return reinterpret_cast<T*>(((unsigned long)hi << 32) | lo);
-}
-
 // A block's columns in registers: rows [w RW, (w+1) RW) of the `rows` below
 // (and with) the block's first pivot row; b[s] = row w RW + 4 s + lk, column li.
 template <int RP>

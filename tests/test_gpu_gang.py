@@ -122,3 +122,28 @@ def test_gang_rank_deficient_panels(env, gang):
     print('  rel.res gang %.2e oracle %.2e' % (res[0] / bn[0], rr), flush=True)
     assert res[0] / bn[0] < 1e-10 and rr < 1e-10
     assert _reldiff(x.cores[:], xr) < 1e-9
+
+
+# both sides of the lines of the on-chip matvec: operator rank (3 and 4) times rows
+# of a member 6 and 8, 9 and 12, members without rows, remainders of the unrolled
+# loads, mode sizes whose pieces fit 136 KB in FP64, in FP32 alone and not at all
+@pytest.mark.parametrize('precision', ['fp64', 'mixed'])
+@pytest.mark.parametrize('d,n,r,gang', [(4, 5, 8, 4), (4, 5, 9, 4), (4, 6, 10, 2), (4, 7, 17, 17), (3, 38, 5, 5),
+                                        (3, 54, 5, 5), (3, 66, 5, 5), (3, 3, 2, 5)])
+def test_gang_few_rows_vs_one_workgroup(env, precision, d, n, r, gang):
+    import scikit_tt_amd.solvers.sle as sle
+    print('case d=%d n=%d r=%d gang=%d %s' % (d, n, r, gang, precision), flush=True)
+    # -Laplacian + its norm: symmetric (CG), condition number below 2, so that local residuals of 1e-12 are local
+    # errors of 2e-12 and the engines' solutions agree to the module's 1e-8; and a non-symmetric one (GMRES)
+    lap = W.tt_sum(W.laplace_operator(d, n), W.identity_operator([n] * d, d * np.linalg.norm(W.laplace_1d(n), 2)))
+    for op in (lap, W.shifted_operator(np.random.default_rng(n), d, n, alpha=10.0 * d)):
+        A = _tt(op)
+        rng = np.random.default_rng(n + r)
+        b = _tt(W.random_tt(rng, [n] * d, 2, scale=1.0 / np.sqrt(n)))
+        ranks = [1] + [min(r, n ** min(k, d - k)) for k in range(1, d)] + [1]
+        x0 = _tt(W.right_orthonormal(W.random_tt(rng, [n] * d, ranks)))
+        (x,), (info,) = sle.als_gang([A], [x0], [b], precision=precision, gang=gang, return_info=True)
+        (y,) = sle.als_batch([A], [x0], [b])
+        assert info.status == 0, info
+        assert x.ranks == y.ranks
+        assert _reldiff(x.cores[:], y.cores[:]) < 1e-8
