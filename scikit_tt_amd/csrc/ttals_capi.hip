@@ -1542,7 +1542,8 @@ struct GangParams {
 
 // Metadata and the gang descriptor of one system (members first .. first+G-1).
 void gang_fill(const GOff& go, const ttals_tt& A, const ttals_tt& x0, const ttals_tt& b, const ttals_tt& xo, int G,
-               int first, const GangParams& P, char* hbase, char* dmeta, char* dbase, GangSync* sync, double* dres,
+               int first, const GangParams& P, char* hbase, char* dmeta, char* dbase, GangSync* sync,
+               unsigned long long* words, double* dres,
                GangDesc& D) {
   const SysOff& o = go.o;
   fill_meta(0, A, x0, &b, xo, o, hbase, dbase);
@@ -1605,6 +1606,7 @@ void gang_fill(const GOff& go, const ttals_tt& A, const ttals_tt& x0, const ttal
   D.qrs = wptr(go.w_qrs);
   D.rmax2 = go.rmax2;
   D.sync = sync;
+  D.words = words;
   D.budget = P.budget;
   D.out = wptr(o.w_out);
   D.res = dres;
@@ -1795,7 +1797,7 @@ int enqueue_hybrid(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, size_t*
   int dmax = 0;
   for (int s = 0; s < count; ++s) dmax = std::max(dmax, B.A[s].order);
   const size_t res_stride = RES_HEAD + (size_t)dmax + 1;
-  const size_t w_sync = dl.take(sizeof(GangSync) * ng);
+  const size_t w_sync = dl.take(gang_sync_bytes(ng, wg));
   const size_t w_res = dl.take(8 * res_stride * count);
   GOff go;
   SysOff o;
@@ -1822,13 +1824,14 @@ int enqueue_hybrid(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, size_t*
   int* hblocks = reinterpret_cast<int*>(hbase + m_blocks);
   SysDesc* hs = reinterpret_cast<SysDesc*>(hbase + m_sdesc);
   GangSync* syncs = reinterpret_cast<GangSync*>(dbase + w_sync);
+  unsigned long long* words = reinterpret_cast<unsigned long long*>(syncs + ng);
   double* dres = reinterpret_cast<double*>(dbase + w_res);
   // pass 2: the same offsets again, descriptors written
   Layout hl2, dl2;
   (void)hl2.take(sizeof(GangDesc) * ng);
   (void)hl2.take(sizeof(int) * wg);
   (void)hl2.take(sizeof(SysDesc) * std::max(nf, 1));
-  (void)dl2.take(sizeof(GangSync) * ng);
+  (void)dl2.take(gang_sync_bytes(ng, wg));
   (void)dl2.take(8 * res_stride * count);
   const GangParams P{B.solver, B.repeats, B.maxit, c->gang_prec, B.tol, c->budget};
   int first = 0;
@@ -1836,7 +1839,7 @@ int enqueue_hybrid(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, size_t*
     const int s = gs[k];
     lay(hl2, dl2, s);
     gang_fill(go, B.A[s], B.x0[s], B.b[s], B.xo[s], G[s], first, P, hbase, dmeta, dbase, syncs + k,
-              dres + res_stride * s, hg[k]);
+              words + 2 * GANG_WORDS * (size_t)first, dres + res_stride * s, hg[k]);
     for (int m = 0; m < G[s]; ++m) hblocks[first + m] = k;
     first += G[s];
   }
@@ -1846,7 +1849,7 @@ int enqueue_hybrid(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, size_t*
     fill_sys(c, B, s, o, hbase, dmeta, dbase, dres + res_stride * s, hs[k]);
   }
   HIPCHK(c, hipMemcpyAsync(dmeta, hbase, meta_bytes, hipMemcpyHostToDevice, stream));
-  HIPCHK(c, hipMemsetAsync(syncs, 0, sizeof(GangSync) * ng, stream));
+  HIPCHK(c, hipMemsetAsync(syncs, 0, gang_sync_bytes(ng, wg), stream));
   if (!c->k0) HIPCHK(c, hipEventCreate(&c->k0));
   if (!c->k1) HIPCHK(c, hipEventCreate(&c->k1));
   {
@@ -1892,7 +1895,7 @@ int gang_solve(ttals_ctx* c, hipStream_t stream, int count, const ttals_tt* A, c
                                     std::to_string(cap));
   const size_t m_blocks = hl.take(sizeof(int) * total);
   const size_t res_stride = RES_HEAD + (size_t)dmax + 1;
-  const size_t w_sync = dl.take(sizeof(GangSync) * count);
+  const size_t w_sync = dl.take(gang_sync_bytes(count, total));
   const size_t w_res = dl.take(8 * res_stride * count);
   GOff go;
   for (int s = 0; s < count; ++s) {
@@ -1911,12 +1914,13 @@ int gang_solve(ttals_ctx* c, hipStream_t stream, int count, const ttals_tt* A, c
   GangDesc* hdesc = reinterpret_cast<GangDesc*>(hbase + m_descs);
   int* hblocks = reinterpret_cast<int*>(hbase + m_blocks);
   GangSync* syncs = reinterpret_cast<GangSync*>(dbase + w_sync);
+  unsigned long long* words = reinterpret_cast<unsigned long long*>(syncs + count);
   double* dres = reinterpret_cast<double*>(dbase + w_res);
   // pass 2: descriptors (same offsets again)
   Layout hl2, dl2;
   (void)hl2.take(sizeof(GangDesc) * count);
   (void)hl2.take(sizeof(int) * total);
-  (void)dl2.take(sizeof(GangSync) * count);
+  (void)dl2.take(gang_sync_bytes(count, total));
   (void)dl2.take(8 * res_stride * count);
   const GangParams P{solver, repeats, maxit, prec, tol, c->budget};
   int first = 0;
@@ -1924,13 +1928,14 @@ int gang_solve(ttals_ctx* c, hipStream_t stream, int count, const ttals_tt* A, c
     (void)size_system(c, 0, A[s], x0[s], &b[s], xo[s], s, z);
     const int G = gang > 0 ? gang : gang_auto_size(x0[s]);
     gang_offsets(z, A[s], x0[s], G, prec == 1, hl2, dl2, go);
-    gang_fill(go, A[s], x0[s], b[s], xo[s], G, first, P, hbase, dmeta, dbase, syncs + s, dres + res_stride * s,
+    gang_fill(go, A[s], x0[s], b[s], xo[s], G, first, P, hbase, dmeta, dbase, syncs + s,
+              words + 2 * GANG_WORDS * (size_t)first, dres + res_stride * s,
               hdesc[s]);
     for (int k = 0; k < G; ++k) hblocks[first + k] = s;
     first += G;
   }
   HIPCHK(c, hipMemcpyAsync(dmeta, hbase, meta_bytes, hipMemcpyHostToDevice, stream));
-  HIPCHK(c, hipMemsetAsync(syncs, 0, sizeof(GangSync) * count, stream));
+  HIPCHK(c, hipMemsetAsync(syncs, 0, gang_sync_bytes(count, total), stream));
   if (!c->k0) HIPCHK(c, hipEventCreate(&c->k0));
   if (!c->k1) HIPCHK(c, hipEventCreate(&c->k1));
   // every workgroup a gang member: k_hybrid with no single-workgroup part

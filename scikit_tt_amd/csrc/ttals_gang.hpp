@@ -33,8 +33,15 @@
 namespace ttals {
 
 struct GangSync {
-  unsigned count, gen, abort, pad;
+  unsigned abort, pad;
 };
+// 64-bit words a member posts at a gang barrier: an epoch in the upper half, a
+// half of one of its (up to two) partial sums in the lower one; two sets, used
+// in turn
+constexpr int GANG_WORDS = 4;
+constexpr size_t gang_sync_bytes(int gangs, int members) {
+  return sizeof(GangSync) * (size_t)gangs + 8 * 2 * GANG_WORDS * (size_t)members;
+}
 
 struct GangDesc {
   int d, solver, repeats, maxit;
@@ -85,6 +92,7 @@ struct GangDesc {
   double* qrs;   // per workgroup: 3 x rmax^2 (Cholesky factor, accumulated R, product)
   long rmax2;    // rmax^2
   GangSync* sync;
+  unsigned long long* words;  // 2 x GANG_WORDS x G, zero at the launch
   long long budget;  // as SysDesc::budget (member 0's clock decides, broadcast at a barrier)
   double* out;   // [16] as SysDesc::out
   double* res;   // compact result row: out[0..15], then the d+1 final ranks
@@ -96,54 +104,90 @@ struct GangDesc {
 // (s_memrealtime): 20 s.  A member may wait for the others to be dispatched
 // while other kernels still hold the CUs, so the bound is in time, not spins.
 constexpr unsigned long long GANG_WAIT_TICKS = 20ull * 100000000ull;
-// partial-sum slots per member: 4 scalars, then two regions of 64 (the two
-// Gram-Schmidt passes of GMRES, KMAX + 2 sums each; the split Householder
-// QR's dots, alternating by column): a member may write one region's sums
-// while another still reads the other's
-constexpr int GANG_LD = 4 + 2 * 64;
+// partial-sum slots per member: two regions of 64 (the two Gram-Schmidt passes
+// of GMRES, KMAX + 2 sums each; the split Householder QR's dots, alternating
+// by column): a member may write one region's sums while another still reads
+// the other's.  Single sums travel with the barrier (gang_sync).
+constexpr int GANG_LD = 2 * 64;
 static_assert(KMAX + 2 <= 64, "a Gram-Schmidt pass's sums fit one region");
 
-// Every workgroup of the gang calls this at the same points.  Returns false
-// once the gang has aborted (a wait ran out): callers then unwind.  Thread 0
-// makes this workgroup's writes visible with ONE release fence, arrives with a
-// relaxed atomic, spins with relaxed loads (an acquire load in the spin would
-// invalidate the caches on every iteration) and acquires once at the end.
-__device__ bool gang_sync(GangSync* s, int G) {
+// Every workgroup of the gang calls this at the same points (epoch counts them,
+// from 1).  Returns false once the gang has aborted (a wait ran out): callers
+// then unwind.  With cnt > 0, out[k] (LDS) is the sum of the members' v_k,
+// in member order, the same bits on every member; buf is LDS for cnt x G.
+// Wave 0 makes this workgroup's writes visible with ONE release fence, posts
+// its words and polls every member's with relaxed loads (an acquire load in
+// the loop would invalidate the caches on every iteration), acquiring once at
+// the end.  A word carries its epoch with its half of the sum, so arrival and
+// sums take one trip through memory; G atomic additions to one counter, the
+// last arrival's release of the others and a read of the sums after that were
+// three (5.6 us against 4.3 us a barrier, 32 members).  A set of words is
+// written again two barriers later, when every member has read it: none
+// passes the next barrier before all have posted there.
+__device__ TT_COLD bool gang_sync(const GangDesc& D, unsigned epoch, int g, int cnt, double v0, double v1, double* buf,
+                                  double* out) {
   __shared__ int ok;
+  GangSync* s = D.sync;
+  const int G = uni(D.G);
+  epoch = uni(epoch);
+  cnt = uni(cnt);
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    unsigned long long* words = D.words + (long)(epoch & 1) * GANG_WORDS * G;
+    const int nw = cnt > 0 ? 2 * cnt : 1;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (lane < nw) {
+      const unsigned long long v = __double_as_longlong((lane >> 1) == 0 ? v0 : v1);
+      __hip_atomic_store(words + lane * G + g, ((unsigned long long)epoch << 32) | (unsigned)(lane & 1 ? v >> 32 : v),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     int good = 1;
-    if (__hip_atomic_load(&s->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-      good = 0;
-    } else {
-      const unsigned gen = __hip_atomic_load(&s->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      const unsigned prev = __hip_atomic_fetch_add(&s->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (prev + 1 == (unsigned)G) {
-        __hip_atomic_store(&s->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&s->gen, gen + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-      } else {
-        const unsigned long long t0 = wall_clock64();
-        unsigned spins = 0;
-        while (__hip_atomic_load(&s->gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gen) {
+    const unsigned long long t0 = wall_clock64();
+    unsigned spins = 0;
+    for (int h0 = 0; h0 < G && good; h0 += 64) {
+      const int h = h0 + lane;
+      unsigned long long x[GANG_WORDS] = {0, 0, 0, 0};
+      for (;;) {
+        bool there = true;
+        if (h < G) {
+#pragma unroll
+          for (int k = 0; k < GANG_WORDS; ++k)
+            if (k < nw) x[k] = __hip_atomic_load(words + k * G + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+          for (int k = 0; k < GANG_WORDS; ++k)
+            if (k < nw) there = there && (unsigned)(x[k] >> 32) == epoch;
+        }
+        if (__ballot(!there) == 0) break;
+        if ((++spins & 15u) == 0) {
           if (__hip_atomic_load(&s->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
             good = 0;
-            break;
-          }
-          if ((++spins & 255u) == 0 && wall_clock64() - t0 > GANG_WAIT_TICKS) {
+          } else if (wall_clock64() - t0 > GANG_WAIT_TICKS) {
             __hip_atomic_store(&s->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             good = 0;
-            break;
           }
-          __builtin_amdgcn_s_sleep(1);
+          good = __builtin_amdgcn_readfirstlane(good);
+          if (!good) break;
         }
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      if (h < G) {
+#pragma unroll
+        for (int k = 0; k < GANG_WORDS / 2; ++k)
+          if (k < cnt) buf[k * G + h] = __longlong_as_double((long long)((x[2 * k + 1] << 32) | (unsigned)x[2 * k]));
+      }
     }
-    ok = good;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (lane == 0) ok = good;
   }
   __syncthreads();
-  return ok != 0;
+  if (threadIdx.x < cnt) {
+    double sg = 0.0;
+    for (int h = 0; h < G; ++h) sg += buf[threadIdx.x * G + h];
+    out[threadIdx.x] = sg;
+  }
+  const bool r = ok != 0;
+  __syncthreads();
+  return r;
 }
 
 // contiguous share [lo, hi) of `total` items for member g of G
@@ -152,7 +196,6 @@ __device__ __forceinline__ void gang_span(int total, int G, int g, int& lo, int&
   hi = (int)((long)total * (g + 1) / G);
 }
 
-// Sum of the G partial sums of slot `k` (stride `ld` per member), same order everywhere.
 // Sums of the G members' partials part[h ld + k0 + k], k < cnt, into out[k]
 // (LDS).  Every load of a round is issued at once -- the partials sit in
 // other members' L2 or in HBM, and G dependent loads would each pay that
@@ -308,9 +351,10 @@ struct GangCtx {
   // bytes per element of the operator pieces held in LDS for the Krylov
   // iterations of the current local problem (gang_op_lds; 0: none)
   int op_lds = 0;
-  __device__ bool sync() {
+  unsigned epoch = 0;  // gang barriers so far
+  __device__ bool sync(int cnt = 0, double v0 = 0.0, double v1 = 0.0, double* out = nullptr) {
     const long long t0 = ph_now();
-    const bool r = gang_sync(D.sync, G);
+    const bool r = gang_sync(D, ++epoch, g, cnt, v0, v1, lds, out);
     ph_add(S, PH_OTHER, t0);  // barrier waits (profiling builds)
     return r;
   }
@@ -364,35 +408,35 @@ __device__ __forceinline__ GangLocal gang_local(const GangCtx& C, int i) {
 
 // LDS of the on-chip matvec of a member with s rows a' (elements of T, after
 // the GEMM staging tiles, which the reductions use): L's rows, the operator
-// core as A'(P, n, m, Q), R, the two intermediates (the first also the result).
+// core as A'(P, n, m, Q), R, the two intermediates and the result.
 template <class T>
 struct GangOpLDS {
-  T *L, *A, *R, *t1, *t2;
+  T *L, *A, *R, *t1, *t2, *y;
   __device__ GangOpLDS(double* lds, int a, int P, int n, int Q, int b, int s) {
     L = reinterpret_cast<T*>(lds + GEMM_LDS_DOUBLES);
     A = L + (long)a * P * s;
     R = A + (long)P * n * n * Q;
     t1 = R + (long)b * Q * b;
-    t2 = t1 + t1_size(s, P, n, b);
-  }
-  static __device__ long t1_size(int s, int P, int n, int b) {
-    const long t1 = ds_t1_size(s, P, n, b), y = (long)s * n * b;
-    return t1 > y ? t1 : y;
+    t2 = t1 + ds_t1_size(s, P, n, b);
+    y = t2 + ds_t2_size(s, n, Q, b);
   }
   static __device__ bool fits(long cap, int a, int P, int n, int Q, int b, int s) {
-    const long e = (long)a * P * s + (long)P * n * n * Q + (long)b * Q * b + t1_size(s, P, n, b) + ds_t2_size(s, n, Q, b);
+    const long e = (long)a * P * s + (long)P * n * n * Q + (long)b * Q * b + ds_t1_size(s, P, n, b) +
+                   ds_t2_size(s, n, Q, b) + (long)s * n * b;
     return P * s <= SKINNY_M && 8 * (cap - GEMM_LDS_DOUBLES) >= (long)sizeof(T) * e;
   }
 };
 
 // Puts the member's operator pieces into LDS for the Krylov iterations of one
-// local problem, where they fit and its rows are few (P s <= SKINNY_M: the
-// first stage keeps one accumulator per row and output column).
+// local problem, where they fit and the rows are few (P s <= SKINNY_M: the
+// first stage keeps one accumulator per row and output column).  Decided for
+// the largest share of rows, so alike in every member: CG's barriers depend
+// on it.
 template <class T>
 __device__ TT_COLD void gang_op_lds(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R) {
   const int s = o.r1 - o.r0;
   C.op_lds = 0;
-  if (s > 0 && GangOpLDS<T>::fits(C.lds_cap, o.a, o.P, o.n, o.Q, o.b, s)) {
+  if (GangOpLDS<T>::fits(C.lds_cap, o.a, o.P, o.n, o.Q, o.b, (o.a + C.G - 1) / C.G)) {
     const GangOpLDS<T> S(C.lds, o.a, o.P, o.n, o.Q, o.b, s);
     const int ps = o.P * s;
     for (int e = threadIdx.x; e < o.a * ps; e += NT) {
@@ -413,59 +457,96 @@ __device__ TT_COLD void gang_op_lds(GangCtx& C, const GangLocal& o, const T* L, 
   __syncthreads();
 }
 
+// V adjacent elements, aligned to V of them
+template <class T, int V>
+struct alignas(sizeof(T) * V) GangPack {
+  T x[V];
+};
+
+// Stage 1 of the on-chip matvec: T1[(a'_l, b), (P, n)] = sum_a L[a, P, r0 + a'_l]
+// v[a, n, b] (+ be T1), a thread per V adjacent columns (n, b), eight loads of
+// v in flight.
+template <class T, int V>
+__device__ __forceinline__ void gang_stage1(int a, int P, int n, int b, int s, const TT_LDS T* Ls, const T* v, TT_LDS T* t1,
+                                            double be) {
+  const int ps = P * s, nb = n * b, s1 = odd_stride(P * n);
+  const float ib = 1.0f / (float)b, is = 1.0f / (float)s;
+  for (int j = V * threadIdx.x; j < nb; j += V * NT) {
+    T acc[SKINNY_M][V];
+#pragma unroll
+    for (int i = 0; i < SKINNY_M; ++i)
+#pragma unroll
+      for (int w = 0; w < V; ++w) acc[i][w] = (T)0;
+    const T* vp = v + j;
+    int k = 0;
+    for (; k + 8 <= a; k += 8) {
+      GangPack<T, V> x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const GangPack<T, V>*>(vp + (k + u) * nb);
+#pragma unroll
+      for (int i = 0; i < SKINNY_M; ++i)
+        if (i < ps) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const T l = Ls[(k + u) * ps + i];
+#pragma unroll
+            for (int w = 0; w < V; ++w) acc[i][w] += l * x[u].x[w];
+          }
+        }
+    }
+    for (; k < a; ++k) {
+      const GangPack<T, V> x = *reinterpret_cast<const GangPack<T, V>*>(vp + k * nb);
+#pragma unroll
+      for (int i = 0; i < SKINNY_M; ++i)
+        if (i < ps) {
+          const T l = Ls[k * ps + i];
+#pragma unroll
+          for (int w = 0; w < V; ++w) acc[i][w] += l * x.x[w];
+        }
+    }
+#pragma unroll
+    for (int w = 0; w < V; ++w) {
+      const int nn = fquot(j + w, ib), bb = j + w - nn * b;
+#pragma unroll
+      for (int i = 0; i < SKINNY_M; ++i)
+        if (i < ps) {
+          const int p = fquot(i, is), al = i - p * s;
+          TT_LDS T* t = t1 + (al * b + bb) * s1 + p * n + nn;
+          *t = be == 0.0 ? acc[i][w] : (T)((double)acc[i][w] + be * (double)*t);
+        }
+    }
+  }
+}
+
 // The member's rows of y = M v with the operator and both intermediates in
 // LDS.  v is read whole (it is complete in global memory), each element once;
 // the contractions after that see no global latency.  The global form
 // (gang_matvec) writes and reads both intermediates through L2 and pays a
 // round trip per K-step of each GEMM: 37.7 ms against 18.9 ms for two sweeps
 // of a system of order 4, n = 32, ranks 32, on 32 members (412 iterations).
+// be != 0: y = M (v + be w) for the w of the call before, whose T1 is still
+// there (stage 1 is linear), so a CG direction needs neither a barrier nor a
+// second vector read.  Reading v is the longest part, 13 us of 19 with 8-byte
+// loads of both v and w: pairs of columns (16 bytes of FP64 a load) of v alone
+// took the same run from 17.8 to 13.8 ms.
 template <class T>
-__device__ TT_COLD void gang_matvec_lds(const GangCtx& C, const GangLocal& o_, const T* v, T* y) {
+__device__ TT_COLD void gang_matvec_lds(const GangCtx& C, const GangLocal& o_, const T* v, T* y, double be) {
   const int a = uni(o_.a), P = uni(o_.P), n = uni(o_.n), Q = uni(o_.Q), b = uni(o_.b), r0 = uni(o_.r0), s = uni(o_.r1) - r0;
   const GangOpLDS<T> S(C.lds, a, P, n, Q, b, s);
-  const int ps = P * s, nb = n * b, s1 = odd_stride(P * n), s2 = odd_stride(b * Q);
-  const TT_LDS T* Ls = (const TT_LDS T*)S.L;
-  TT_LDS T* t1 = (TT_LDS T*)S.t1;
-  const float ib = 1.0f / (float)b, is = 1.0f / (float)s;
-  // T1[(a'_l, b), (P, n)] = sum_a L[a, P, r0 + a'_l] v[a, n, b]: a thread per
-  // column (n, b), eight loads of v in flight
-  for (int j = threadIdx.x; j < nb; j += NT) {
-    T acc[SKINNY_M];
-#pragma unroll
-    for (int i = 0; i < SKINNY_M; ++i) acc[i] = (T)0;
-    const T* vp = v + j;
-    int k = 0;
-    for (; k + 8 <= a; k += 8) {
-      T x[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = vp[(long)(k + u) * nb];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int i = 0; i < SKINNY_M; ++i)
-          if (i < ps) acc[i] += Ls[(k + u) * ps + i] * x[u];
-    }
-    for (; k < a; ++k) {
-      const T x = vp[(long)k * nb];
-#pragma unroll
-      for (int i = 0; i < SKINNY_M; ++i)
-        if (i < ps) acc[i] += Ls[k * ps + i] * x;
-    }
-    const int nn = fquot(j, ib), bb = j - nn * b;
-#pragma unroll
-    for (int i = 0; i < SKINNY_M; ++i)
-      if (i < ps) {
-        const int p = fquot(i, is), al = i - p * s;
-        t1[(al * b + bb) * s1 + p * n + nn] = acc[i];
-      }
-  }
+  if (s == 0) return;
+  const int nb = n * b, s1 = odd_stride(P * n), s2 = odd_stride(b * Q);
+  if ((nb & 1) == 0 && (reinterpret_cast<size_t>(v) & (2 * sizeof(T) - 1)) == 0)
+    gang_stage1<T, 2>(a, P, n, b, s, (const TT_LDS T*)S.L, v, (TT_LDS T*)S.t1, be);
+  else
+    gang_stage1<T, 1>(a, P, n, b, s, (const TT_LDS T*)S.L, v, (TT_LDS T*)S.t1, be);
   __syncthreads();
   // T2[(a'_l, m), (b, Q)] and y[(a'_l, m), b'] as on-chip matrix-core GEMMs
   mf_gemm_lin<T>(s * b, n * Q, P * n, S.t1, s1, 1, S.A, n * Q, 1, S.t2, fmap(b, n * s2, Q), fmap(Q, s2, 1), (T*)nullptr,
                  0);
-  mf_gemm_lin<T>(s * n, b, b * Q, S.t2, s2, 1, S.R, b, 1, S.t1, fmap(1, b, 0), fmap(1, 1, 0), (T*)nullptr, 0);
+  mf_gemm_lin<T>(s * n, b, b * Q, S.t2, s2, 1, S.R, b, 1, S.y, fmap(1, b, 0), fmap(1, 1, 0), (T*)nullptr, 0);
   T* yo = y + (long)r0 * nb;
-  for (int e = threadIdx.x; e < s * nb; e += NT) yo[e] = t1[e];
+  const TT_LDS T* yl = (const TT_LDS T*)S.y;
+  for (int e = threadIdx.x; e < s * nb; e += NT) yo[e] = yl[e];
   __syncthreads();
 }
 
@@ -473,7 +554,7 @@ template <class T>
 __device__ __forceinline__ void gang_apply(const GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R,
                                            const T* v, T* y) {
   if (C.op_lds == (int)sizeof(T))
-    gang_matvec_lds<T>(C, o, v, y);
+    gang_matvec_lds<T>(C, o, v, y, 0.0);
   else
     gang_matvec<T>(o.a, o.P, o.n, o.Q, o.b, L, A, R, v, y, o.r0, o.r1, reinterpret_cast<T*>(C.t1),
                    reinterpret_cast<T*>(C.t2), reinterpret_cast<T*>(C.lds));
@@ -482,12 +563,14 @@ __device__ __forceinline__ void gang_apply(const GangCtx& C, const GangLocal& o,
 // Conjugate gradients on M x = f (x holds the start), vectors of type T,
 // matvec on operands (L, A, R) of type T, reductions in FP64.  Returns 0
 // converged, 1 p^T M p <= 0 (not SPD), 2 maxit, -1 gang aborted.
+// An iteration has a barrier for each of its two sums.  A third one completes
+// the direction where the matvec reads it from global memory; the on-chip
+// matvec reads the residual, complete by then, and adds the last direction's
+// first contraction, which it still holds.
 template <class T>
 __device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R, T* x, const T* f, T* r,
                        T* p, T* q, double tol, int maxit, int* iters, double* vfl) {
-  const int G = C.G, g = C.g;
-  const int ld = GANG_LD;
-  double* part = C.D.part;
+  const bool split = C.op_lds == (int)sizeof(T);
   // r = f - M x, p = r; |f|, |r|
   gang_apply<T>(C, o, L, A, R, x, q);
   double ff = 0.0, rr = 0.0;
@@ -500,30 +583,27 @@ __device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const
   }
   double d1 = 0.0;
   wg_sum3(ff, rr, d1, C.S.red);
-  if (threadIdx.x == 0) {
-    part[(long)g * ld + 0] = ff;
-    part[(long)g * ld + 1] = rr;
-  }
-  if (!C.sync()) return -1;
   double* tot = C.S.scal + 2;  // two LDS slots for scalar totals
-  gang_totals(part, G, ld, 0, 2, C.lds, tot);
+  if (!C.sync(2, ff, rr, tot)) return -1;
   ff = tot[0];
   rr = tot[1];
   const double fn = sqrt(ff);
   if (threadIdx.x == 0) *vfl += 4.0 * o.N;
   if (fn == 0.0 || sqrt(rr) <= tol * fn) return 0;
+  double be = 0.0;
   while (*iters < maxit) {
     // q = M p (p complete: the barrier above / at the end of the last step)
     const long long tm = ph_now();
-    gang_apply<T>(C, o, L, A, R, p, q);
+    if (split)  // the first direction is the residual
+      gang_matvec_lds<T>(C, o, r, q, be);
+    else
+      gang_apply<T>(C, o, L, A, R, p, q);
     ph_add(C.S, PH_MATVEC, tm);
     double pq = 0.0;
     for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) pq += (double)p[e] * (double)q[e];
     double u1 = 0.0, u2 = 0.0;
     wg_sum3(pq, u1, u2, C.S.red);
-    if (threadIdx.x == 0) part[(long)g * ld + 2] = pq;
-    if (!C.sync()) return -1;
-    gang_totals(part, G, ld, 2, 1, C.lds, tot);
+    if (!C.sync(1, pq, 0.0, tot)) return -1;
     pq = tot[0];
     if (!(pq > 0.0)) return 1;
     const double al = rr / pq;
@@ -535,17 +615,15 @@ __device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const
       rn += re * re;
     }
     wg_sum3(rn, u1, u2, C.S.red);
-    if (threadIdx.x == 0) part[(long)g * ld + 3] = rn;
-    if (!C.sync()) return -1;
-    gang_totals(part, G, ld, 3, 1, C.lds, tot);
+    if (!C.sync(1, rn, 0.0, tot)) return -1;
     rn = tot[0];
     ++*iters;
     if (threadIdx.x == 0) *vfl += 10.0 * o.N;
     if (sqrt(rn) <= tol * fn) return 0;
-    const double be = rn / rr;
+    be = rn / rr;
     rr = rn;
     for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) p[e] = (T)((double)r[e] + be * (double)p[e]);
-    if (!C.sync()) return -1;
+    if (!split && !C.sync()) return -1;
   }
   return 2;
 }
@@ -570,10 +648,8 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
   for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) ff += (double)f[e] * (double)f[e];
   double u1 = 0.0, u2 = 0.0;
   wg_sum3(ff, u1, u2, S.red);
-  if (threadIdx.x == 0) part[(long)g * ld + 0] = ff;
-  if (!C.sync()) return -1;
   double* tot = S.scal + 2;  // two LDS slots for scalar totals (S.scal[0] is the Givens residual)
-  gang_totals(part, G, ld, 0, 1, C.lds, tot);
+  if (!C.sync(1, ff, 0.0, tot)) return -1;
   const double fn = sqrt(tot[0]);
   if (fn == 0.0) {
     for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) x[e] = (T)0;
@@ -589,9 +665,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
       bb += we * we;
     }
     wg_sum3(bb, u1, u2, S.red);
-    if (threadIdx.x == 0) part[(long)g * ld + 1] = bb;
-    if (!C.sync()) return -1;
-    gang_totals(part, G, ld, 1, 1, C.lds, tot);
+    if (!C.sync(1, bb, 0.0, tot)) return -1;
     const double beta = sqrt(tot[0]);
     if (threadIdx.x == 0) *vfl += 4.0 * N;
     if (beta <= tol * fn) return 0;
@@ -615,7 +689,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
       double w0 = 0.0, hn = 0.0;
       for (int pass = 0; pass < 2; ++pass) {
         // partial dots <V_k, w> over this member's elements, k <= j, and |w|^2
-        const int base = 4 + pass * (KMAX + 2);
+        const int base = pass * (KMAX + 2);
         gang_multidot<T>(V, N, j + 1, w, o.e0, o.e1, part + (long)g * ld + base, S.part);
         if (!C.sync()) return -1;
         gang_totals(part, G, ld, base, j + 2, C.lds, S.h);
@@ -633,9 +707,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
       double ww = 0.0;
       for (long e = o.e0 + threadIdx.x; e < o.e1; e += NT) ww += (double)w[e] * (double)w[e];
       ww = wg_sum(ww, S.red);
-      if (threadIdx.x == 0) part[(long)g * ld + 2] = ww;
-      if (!C.sync()) return -1;
-      gang_totals(part, G, ld, 2, 1, C.lds, tot);
+      if (!C.sync(1, ww, 0.0, tot)) return -1;
       hn = sqrt(tot[0]);
       if (!(hn > 1e-14 * w0)) {
         hn = 0.0;  // (lucky) breakdown: the Krylov space is invariant
@@ -704,9 +776,7 @@ __device__ TT_COLD int gang_gmres(GangCtx& C, const GangLocal& o, const T* L, co
         tr += we * we;
       }
       tr = wg_sum(tr, S.red);
-      if (threadIdx.x == 0) part[(long)g * ld + 1] = tr;
-      if (!C.sync()) return -1;
-      gang_totals(part, G, ld, 1, 1, C.lds, tot);
+      if (!C.sync(1, tr, 0.0, tot)) return -1;
       return sqrt(tot[0]) <= tol * fn ? 0 : 2;
     }
   }
@@ -961,15 +1031,7 @@ __device__ TT_COLD int gang_hhqr(GangCtx& C, const double* g, int m, int c, bool
     }
     if (threadIdx.x == 0 && j >= m0 && j < m1) al = W[(long)j * c + j];
     wg_sum3(s2, al, u, S.red);
-    // slots alternate by column: when column j has no reflector there is no
-    // second barrier before column j + 1 writes its sums
-    const int ns = 2 * (j & 1);
-    if (threadIdx.x == 0) {
-      part[(long)C.g * ld + ns] = s2;
-      part[(long)C.g * ld + ns + 1] = al;
-    }
-    if (!C.sync()) return -1;
-    gang_totals(part, G, ld, ns, 2, C.lds, tot);
+    if (!C.sync(2, s2, al, tot)) return -1;
     s2 = tot[0];
     const double alpha = tot[1];
     double t = 0.0;
@@ -987,7 +1049,7 @@ __device__ TT_COLD int gang_hhqr(GangCtx& C, const double* g, int m, int c, bool
     if (t != 0.0 && nq > 0) {
       const int lo = m0 > j ? m0 : j;
       rows_dots(W, W, c, j, lo, m1, j + 1, nq, C.lds, wv);
-      const int rg = 4 + 64 * (j & 1);
+      const int rg = 64 * (j & 1);
       for (int q = threadIdx.x; q < nq; q += NT) part[(long)C.g * ld + rg + q] = wv[q];
       if (!C.sync()) return -1;
       gang_totals(part, G, ld, rg, nq, C.lds, wv);
@@ -1018,7 +1080,7 @@ __device__ TT_COLD int gang_hhqr(GangCtx& C, const double* g, int m, int c, bool
     const int lo = m0 > j ? m0 : j;
     rows_dots(W, Qm, c, j, lo, m1, j, nq, C.lds, wv);
     // one barrier per column: consecutive columns use the two regions in turn
-    const int rg = 4 + 64 * (qcount++ & 1);
+    const int rg = 64 * (qcount++ & 1);
     for (int q = threadIdx.x; q < nq; q += NT) part[(long)C.g * ld + rg + q] = wv[q];
     if (!C.sync()) return -1;
     gang_totals(part, G, ld, rg, nq, C.lds, wv);
@@ -1237,7 +1299,7 @@ __device__ TT_COLD bool gang_ortho_right(GangCtx& C, double* fl) {
 // One local step at position i: local rhs, the split Krylov solve (FP64, or
 // FP32 with FP64 refinement), then on member 0 the QR of the new core, the
 // core store and the warm start of the next position.  Returns a Status.
-__device__ int gang_step(GangCtx& C, int i, bool forward, bool sym, StepStats& st) {
+__device__ TT_COLD int gang_step(GangCtx& C, int i, bool forward, bool sym, StepStats& st) {
   const GangDesc& D = C.D;
   SolveLDS& S = C.S;
   const GangLocal o = gang_local(C, i);
@@ -1287,13 +1349,7 @@ __device__ int gang_step(GangCtx& C, int i, bool forward, bool sym, StepStats& s
         rr += re * re;
       }
       wg_sum3(ff, rr, mx, S.red);
-      const int ld = GANG_LD;
-      if (threadIdx.x == 0) {
-        D.part[(long)C.g * ld + 0] = ff;
-        D.part[(long)C.g * ld + 1] = rr;
-      }
-      if (!C.sync()) return ST_ABORT;
-      gang_totals(D.part, C.G, ld, 0, 2, C.lds, S.scal + 2);
+      if (!C.sync(2, ff, rr, S.scal + 2)) return ST_ABORT;
       const double fn = sqrt(S.scal[2]), rn = sqrt(S.scal[3]);
       vfl += 5.0 * o.N;
       st.flops += fmv;

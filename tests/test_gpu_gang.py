@@ -128,7 +128,7 @@ def test_gang_rank_deficient_panels(env, gang):
 # of a member 6 and 8, 9 and 12, members without rows, remainders of the unrolled
 # loads, mode sizes whose pieces fit 136 KB in FP64, in FP32 alone and not at all
 @pytest.mark.parametrize('precision', ['fp64', 'mixed'])
-@pytest.mark.parametrize('d,n,r,gang', [(4, 5, 8, 4), (4, 5, 9, 4), (4, 6, 10, 2), (4, 7, 17, 17), (3, 38, 5, 5),
+@pytest.mark.parametrize('d,n,r,gang', [(4, 5, 8, 4), (4, 5, 9, 4), (4, 6, 10, 2), (4, 7, 17, 17), (3, 36, 5, 5),
                                         (3, 54, 5, 5), (3, 66, 5, 5), (3, 3, 2, 5)])
 def test_gang_few_rows_vs_one_workgroup(env, precision, d, n, r, gang):
     import scikit_tt_amd.solvers.sle as sle
