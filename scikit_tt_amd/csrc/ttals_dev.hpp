@@ -329,15 +329,6 @@ __device__ __forceinline__ int mfma16_row(int lk, int e) {
   return std::is_same<T, double>::value ? lk + 4 * e : 4 * lk + e;
 }
 
-// K-steps of operands in flight during a K-step's MFMAs: 1 where the kernel
-// must stay within 256 registers for two workgroups per CU (k_als), 2 in a
-// translation unit that defines TTALS_GEMM_PREFETCH for a one-workgroup-per-CU
-// kernel (the same arithmetic either way).
-#ifndef TTALS_GEMM_PREFETCH
-#define TTALS_GEMM_PREFETCH 1
-#endif
-constexpr int GEMM_PREFETCH = TTALS_GEMM_PREFETCH;
-
 // FP64 GEMM over global (L2/HBM) operands on the matrix cores.  GBM x 64 output
 // tiles, K-steps of 16 staged through LDS ([GBK][GBM+1] and [GBK][GBN+1]:
 // the odd stride keeps the transposing stores of k-fast operands off a single
@@ -411,8 +402,14 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int g = 0; g < 2; ++g) acc[h][g] = acc_t{0, 0, 0, 0};
-  // the MFMAs of the staged K-step, and the tile's store after its last one
-  auto compute = [&]() {
+  T ra[4], rb[NB_LD];
+  if (steps > 0) {
+    load(ra, rb);
+    stage(ra, rb);
+  }
+  __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    if (s + 1 < steps) load(ra, rb);
 #pragma unroll
     for (int q = 0; q < GBK / 4; ++q) {
       const int kr = (4 * q + lk);
@@ -450,81 +447,10 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
         cm0 += GBM;
       }
     }
-  };
-  if constexpr (GEMM_PREFETCH == 2) {
-    // two register sets: while step s computes, steps s+1 and s+2 are loading
-    T ra0[4], rb0[NB_LD], ra1[4], rb1[NB_LD];
-    if (steps > 0) {
-      load(ra0, rb0);
-      stage(ra0, rb0);
-    }
-    if (steps > 1) load(ra1, rb1);
     __syncthreads();
-    for (int s = 0; s < steps; s += 2) {
-      if (s + 2 < steps) load(ra0, rb0);
-      compute();
-      __syncthreads();
-      if (s + 1 >= steps) break;
-      stage(ra1, rb1);
-      __syncthreads();
-      if (s + 3 < steps) load(ra1, rb1);
-      compute();
-      __syncthreads();
-      if (s + 2 < steps) {
-        stage(ra0, rb0);
-        __syncthreads();
-      }
-    }
-  } else {
-    T ra[4], rb[NB_LD];
-    if (steps > 0) {
-      load(ra, rb);
+    if (s + 1 < steps) {
       stage(ra, rb);
-    }
-    __syncthreads();
-    for (int s = 0; s < steps; ++s) {
-      if (s + 1 < steps) load(ra, rb);
-#pragma unroll
-      for (int q = 0; q < GBK / 4; ++q) {
-        const int kr = (4 * q + lk);
-        const T a0 = As[kr * (GBM + 1) + wm + li], a1 = As[kr * (GBM + 1) + wm + 16 + li];
-        const T b0 = Bs[kr * (GBN + 1) + wn + li], b1 = Bs[kr * (GBN + 1) + wn + 16 + li];
-        acc[0][0] = mfma16x16x4(a0, b0, acc[0][0]);
-        acc[0][1] = mfma16x16x4(a0, b1, acc[0][1]);
-        acc[1][0] = mfma16x16x4(a1, b0, acc[1][0]);
-        acc[1][1] = mfma16x16x4(a1, b1, acc[1][1]);
-      }
-      ckk += GBK;
-      if (ckk >= K) {
-        const GMap Cr = gmap(C.r), Cc = gmap(C.c);
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          const int gn = cn0 + wn + 16 * g + li;
-          const bool nv = gn < N;
-          const int cc = nv ? gmap_at(Cc, gn) : 0;
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int gm = cm0 + wm + 16 * h + mfma16_row<T>(lk, e);
-              if (nv && gm < M) C.p[gmap_at(Cr, gm) + cc] = acc[h][g][e];
-            }
-            acc[h][g] = acc_t{0, 0, 0, 0};
-          }
-        }
-        ckk = 0;
-        cn0 += GBN;
-        if (++ctj == tn) {
-          ctj = 0;
-          cn0 = 0;
-          cm0 += GBM;
-        }
-      }
       __syncthreads();
-      if (s + 1 < steps) {
-        stage(ra, rb);
-        __syncthreads();
-      }
     }
   }
 }
@@ -1787,8 +1713,8 @@ __device__ void hh_block_t(const double* tau, const double* G, int kb, double* T
 // memory latency, not arithmetic).  Partial Y meet within the wave by lane
 // exchanges and across the waves in Yb (NB x 64 doubles), in a fixed order.
 // HH_U: 2 where the kernel must stay within 256 registers for two workgroups
-// per CU (k_als), 8 in a translation unit that defines TTALS_HH_ROWS for a
-// one-workgroup-per-CU kernel.
+// per CU (k_als), 4 in a translation unit that defines TTALS_HH_ROWS for a
+// one-workgroup-per-CU kernel .
 #ifndef TTALS_HH_ROWS
 #define TTALS_HH_ROWS 2
 #endif

@@ -1,11 +1,12 @@
 // k_hybrid: one launch that mixes gangs and single-workgroup systems.
 //
-// A translation unit of its own: the engine's out-of-line device functions
-// are compiled here for k_hybrid's occupancy (one workgroup per CU, set by
-// the gang path's registers), while k_als keeps its own copies, compiled for
-// two resident workgroups per CU.  With registers to spare, the blocked
-// QR's streaming passes keep eight rows per lane in flight and the global
-// GEMMs two K-steps (same arithmetic order as k_als's two rows and one step).
+// A translation unit of its own: the engine's device functions are compiled
+// here for one workgroup of eight waves per CU (the gang path's registers and
+// a large arena leave no room for a second one), while k_als keeps its own
+// copies, compiled for two resident workgroups of four.  Eight waves hide
+// about twice the latency of four: 512 mixed systems, orders 8..24 and ranks
+// up to 48, 84 ms with four waves, 78 with eight.  With registers to spare,
+// the blocked QR's streaming passes keep four rows per lane in flight.
 #define TTALS_NT 512
 #define TTALS_HH_ROWS 4
 #include "ttals_hybrid.hpp"
