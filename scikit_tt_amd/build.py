@@ -7,7 +7,8 @@ import sys
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRCS = [os.path.join(HERE, 'csrc', f) for f in ('ttals_capi.hip', 'ttals_hybrid.hip', 'ttals_tt.hip')]
+SRCS = [os.path.join(HERE, 'csrc', f) for f in ('ttals_capi.hip', 'ttals_hybrid.hip', 'ttals_piece.hip',
+                                                'ttals_tt.hip')]
 OUT = os.path.join(HERE, 'libttals.so')
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC',

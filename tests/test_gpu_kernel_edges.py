@@ -168,6 +168,69 @@ def test_local_lu(lib, a, P, n, Q, b, kb):
     assert res <= 4 * N * N * EPS * float(M.norm()) * float(v.norm())
 
 
+# (a, P, n, Q, b): a local problem in 61 KB, two in the CU's LDS alone, two in
+# neither (all but the first on eight waves); uneven ranks, odd sizes
+PIECES = [(8, 2, 10, 2, 8), (9, 2, 10, 2, 10), (8, 3, 17, 2, 8), (8, 2, 33, 2, 8), (5, 1, 40, 3, 12)]
+
+
+@pytest.mark.parametrize('a,P,n,Q,b', PIECES)
+def test_pieces_of_local_problems(lib, a, P, n, Q, b):
+    """Matvec and left interface update against torch, the local solves by
+    their residual (both iterations stop at 1e-11), the lowest eigenvalue
+    against a dense eigensolver (residual 1e-11 of the norm bounds its error).
+    Operator: twice the identity plus a symmetric part of norm below 1/2."""
+    from scikit_tt_amd import _lib
+    gen = torch.Generator(device='cuda').manual_seed(a * 1000 + n)
+
+    def sym(x):
+        x = x + x.transpose(0, -1)
+        return x / (P * Q * 2.0 * torch.linalg.matrix_norm(x.permute(1, 0, 2), 2).max())
+
+    L, R, A = _randn(gen, a, P, a), _randn(gen, b, Q, b), _randn(gen, P, n, n, Q)
+    L = sym(L)
+    R = sym(R)
+    A = A + A.transpose(1, 2)
+    A = A / torch.linalg.matrix_norm(A.permute(0, 3, 1, 2), 2).max()
+    L[:, 0, :] = torch.eye(a, device='cuda', dtype=torch.float64)
+    R[:, 0, :] = torch.eye(b, device='cuda', dtype=torch.float64)
+    A[0, :, :, 0] = 2.0 * torch.eye(n, device='cuda', dtype=torch.float64)
+    L, R, A = L.contiguous(), R.contiguous(), A.contiguous()
+    N = a * n * b
+    f, x = _randn(gen, N), _randn(gen, N)
+
+    def chain(l, o, r, v):
+        t = torch.tensordot(l, v.view(a, n, b), dims=([0], [0]))  # P a' n b
+        t = torch.tensordot(t, o, dims=([0, 2], [0, 2]))          # a' b m Q
+        return torch.tensordot(t, r, dims=([1, 3], [0, 1])).reshape(N)
+
+    def left(l, o, v):
+        t = torch.tensordot(l, v.view(a, n, b), dims=([0], [0]))
+        t = torch.tensordot(t, o, dims=([0, 2], [0, 2]))
+        return torch.tensordot(t, v.view(a, n, b), dims=([0, 2], [0, 1])).contiguous()  # b Q b'
+
+    ctx = _lib.context(0)
+    y = torch.empty(N, dtype=torch.float64, device='cuda')
+    assert lib.ttals_micro_matvec(ctx, None, a, P, n, Q, b, _ptr(L), _ptr(A), _ptr(R), _ptr(x), _ptr(y)) == 0
+    terms = (a + P * n + b * Q + 3) * EPS
+    assert bool(((y - chain(L, A, R, x)).abs() <= 2 * terms * chain(L.abs(), A.abs(), R.abs(), x.abs())).all())
+    out = torch.empty(b, Q, b, dtype=torch.float64, device='cuda')
+    assert lib.ttals_stack_left_op(ctx, None, a, P, n, Q, b, _ptr(L), _ptr(A), _ptr(x), _ptr(out)) == 0
+    bound = 2 * (a + P * n + a * n + 3) * EPS * left(L.abs(), A.abs(), x.abs())
+    assert bool(((out - left(L, A, x)).abs() <= bound).all())
+    for method in (2, 3):
+        v, its = torch.zeros_like(f), ctypes.c_int()
+        assert lib.ttals_local_solve(ctx, None, a, P, n, Q, b, _ptr(L), _ptr(A), _ptr(R), _ptr(f), _ptr(v), method, 1,
+                                     1e-11, 400, ctypes.byref(its)) == 0
+        assert float((chain(L, A, R, v) - f).norm()) <= 2e-11 * float(f.norm())
+    lam, its = ctypes.c_double(), ctypes.c_int()
+    v = f.clone()
+    assert lib.ttals_local_eig(ctx, None, a, P, n, Q, b, _ptr(L), _ptr(A), _ptr(R), _ptr(v), 0, 0.0, 1e-11, 4000,
+                               ctypes.byref(lam), ctypes.byref(its)) == 0
+    M = torch.stack([chain(L, A, R, e) for e in torch.eye(N, dtype=torch.float64, device='cuda')])
+    want = float(torch.linalg.eigvalsh(0.5 * (M + M.T))[0])
+    assert abs(lam.value - want) <= 1e-10 * float(M.norm())
+
+
 def test_one_schedule_result_does_not_depend_on_the_batch(lib):
     """Systems on both sides of the line between the two single-workgroup
     kernels (10240 unknowns): in one batch, in another order and alone, the
