@@ -95,7 +95,9 @@ int ttals_set_trace(ttals_ctx* ctx, double* buf, long long cap);
 /* ---- whole solvers (synchronous: return when the results are on the host) */
 
 /* Replaces scikit_tt.solvers.sle.als (scikit_tt/solvers/sle.py:10-95) for
- * `count` independent systems in ONE launch (one workgroup per system).
+ * `count` independent systems in one submission (one workgroup per system;
+ * systems with a local problem of 10240 unknowns or more in a launch of wider
+ * workgroups beside the others').
  * solver: 0 = 'solve', 1 = 'lu' (both: LU for local size <= 96, matrix-free
  * CG/GMRES above).  tol/maxit: local Krylov relative tolerance / cap.
  * x_out[s] receives the solution (cores in place, final ranks). */

@@ -1190,6 +1190,69 @@ __device__ int gang_hhqr_run(GangCtx& C, int m, int c) {
   return 0;
 }
 
+// The split QR with the register-blocked factorisation (ttals_qr.hpp): every
+// member copies each block of 16 columns to its own scratch (t1) and factors
+// it there, updates its share of the trailing columns, and applies the blocks
+// to its share of Q's columns, which needs no exchange.  Half the blocks and
+// barriers of the form above, and none of its reductions through LDS.  Panels
+// whose rows exceed the registers (2304) or whose copy exceeds the scratch keep
+// that form.  512 mixed systems with rank-deficient panels, orders 8..24, ranks
+// up to 48: the largest alone on gangs of 2 / 4 / 8 70.5 / 52.2 / 44.0 ms with
+// the LDS blocks, 58.1 / 40.9 / 33.1 ms here; the batch 75.0 and 70.0 ms.
+__device__ __forceinline__ bool gang_hq_fits(const GangCtx& C, int m, int c) {
+  const long cr = (c + HQ_NB - 1) / HQ_NB * HQ_NB;
+  return m <= HQ_ROWS_MAX && hq_fits(m, c) && (long)sizeof(HqLDS) <= 8 * C.lds_cap && m * cr <= C.D.tmax &&
+         HQ_NB * cr <= C.D.tmax;
+}
+__device__ __forceinline__ int gang_hq_run(GangCtx& C, int m, int c) {
+  const GangDesc& D = C.D;
+  const HqL S = (HqL)C.lds;
+  double *W = D.qw, *V = C.t1, *T = C.t2, *Q = D.qq;
+  for (int jb = 0; jb < c; jb += HQ_NB) {
+    const int kb = min(HQ_NB, c - jb), rows = m - jb, c2 = c - jb - kb;
+    double* Vb = V + (long)jb * m;
+    for (int e = threadIdx.x; e < rows * HQ_NB; e += NT) {
+      const int i = e / HQ_NB, q = e % HQ_NB;
+      if (q < kb) Vb[e] = W[(long)(jb + i) * c + jb + q];
+    }
+    __syncthreads();
+    double* Tb = T + jb * HQ_NB;
+    hq_dispatch(rows, [&](auto RPc) { hq_block<decltype(RPc)::value>(Vb, HQ_NB, rows, kb, Tb, S); });
+    if (c2 > 0) {
+      int j0, j1;
+      gang_span(c2, C.G, C.g, j0, j1);
+      if (j1 > j0) hq_apply(Vb, HQ_NB, kb, W + (long)jb * c + jb + kb + j0, c, rows, j1 - j0, true, S);
+      if (!C.sync()) return -1;  // the next block's columns complete
+    }
+  }
+  // member 0: R, its diagonal blocks from the factored ones
+  if (C.g == 0) {
+    for (int e = threadIdx.x; e < c * c; e += NT) {
+      const int i = e / c, j = e - i * c, jb = j / HQ_NB * HQ_NB;
+      D.rf[e] = j < i ? 0.0 : (i < jb ? W[e] : V[(long)jb * m + (i - jb) * HQ_NB + (j - jb)]);
+    }
+  }
+  // this member's columns of Q
+  int j0, j1;
+  gang_span(c, C.G, C.g, j0, j1);
+  const int nc = j1 - j0;
+  if (nc > 0) {
+    for (int e = threadIdx.x; e < m * nc; e += NT) {
+      const int i = e / nc, j = j0 + e - i * nc;
+      Q[(long)i * c + j] = i == j ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    for (int jb = (j1 - 1) / HQ_NB * HQ_NB; jb >= 0; jb -= HQ_NB) {
+      const int x0 = max(j0, jb);
+      for (int e = threadIdx.x; e < HQ_NB * HQ_NB; e += NT) S->T[e >> 4][e & 15] = T[jb * HQ_NB + e];
+      __syncthreads();
+      hq_apply(V + (long)jb * m, HQ_NB, min(HQ_NB, c - jb), Q + (long)jb * c + x0, c, m - jb, j1 - x0, false, S);
+    }
+  }
+  __syncthreads();
+  return 0;
+}
+
 __device__ TT_COLD int gang_hhqr_blocked(GangCtx& C, const double* g, int m, int c, bool transposed, double* fl,
                                  const double** Qout, const double** Rout) {
   const GangDesc& D = C.D;
@@ -1202,7 +1265,8 @@ __device__ TT_COLD int gang_hhqr_blocked(GangCtx& C, const double* g, int m, int
   __syncthreads();
   if (!C.sync()) return -1;
   const long lim = C.lds_cap < HHQR_LDS_CAP ? C.lds_cap : HHQR_LDS_CAP;
-  const int r = HHBlockLDS<8>::need(m) <= lim ? gang_hhqr_run<8>(C, m, c) : gang_hhqr_run<4>(C, m, c);
+  const int r = gang_hq_fits(C, m, c) ? gang_hq_run(C, m, c)
+                : HHBlockLDS<8>::need(m) <= lim ? gang_hhqr_run<8>(C, m, c) : gang_hhqr_run<4>(C, m, c);
   if (r < 0) return -1;
   if (!C.sync()) return -1;  // Q rows and R complete
   *fl += 4.0 * (double)m * c * c - 4.0 / 3.0 * (double)c * c * c;

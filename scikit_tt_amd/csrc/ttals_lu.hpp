@@ -1,6 +1,6 @@
 // Dense local solve in registers: the micro matrix of a local linear system
-// of at most 64 unknowns (96 with eight waves) is assembled straight into registers and solved by
-// LU with partial pivoting, one workgroup.
+// of at most 64 unknowns (96 with eight waves) is assembled straight into
+// registers and solved by LU with partial pivoting, one workgroup.
 //
 // What bounds it: N dependent elimination steps.  Lane = matrix row (two rows
 // past 64), each wave a block of CB columns in registers, so a step is one

@@ -8,7 +8,8 @@
 // one barrier instead of by global memory latency per column element, and the
 // final sort counts ranks in parallel instead of selecting on one thread.
 // An 80 x 80 triangular factor of a rounding sweep: 5.5 ms in global memory
-// with one wave per pair, 0.8 ms here.
+// with one wave per pair, 0.8 ms here; one root and one division a rotation
+// then took a 64 x 64 one from 1.00 to 0.73 ms.
 #pragma once
 #include "ttals_dev.hpp"
 #include "ttals_qr.hpp"

@@ -4,7 +4,7 @@ Requests (``sle.als`` or ``evp.als`` problems whose TTs already live on the
 device) are queued on arrival.  The loop keeps ``slots`` engine contexts,
 each with its own HIP stream and workspace.  Whenever a slot is free it
 admits the waiting requests of one kind/parameter set (FIFO, up to
-``max_batch`` and within the HBM budget) as ONE launch.  Launches on
+``max_batch`` and within the HBM budget) as ONE submission.  Launches on
 different slots run concurrently on the device, so requests that arrive
 while others are on the GPU start as soon as a slot and memory free up
 instead of waiting for the running batch.  Cores and stacks stay resident on

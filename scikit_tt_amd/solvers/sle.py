@@ -4,7 +4,8 @@ Drop-in for scikit_tt.solvers.sle.als (scikit_tt/solvers/sle.py:10-95): same
 signature, defaults and return convention (a new TT with cores
 ``(r_i, n_i, 1, r_{i+1})``, cores 1..d-1 right-orthonormal, the norm in core
 0).  One call is one launch of the fused engine in libttals.so; ``als_batch``
-solves many independent systems of uneven order and rank in one launch.
+solves many independent systems of uneven order and rank in one launch (two
+side by side where some have local problems of 10240 unknowns or more).
 
 Local solves: LU with partial pivoting (as dgesv, sle.py:506) for local size
 <= 96, matrix-free CG (operator symmetric slice by slice; falls back to

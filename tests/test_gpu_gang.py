@@ -147,3 +147,27 @@ def test_gang_few_rows_vs_one_workgroup(env, precision, d, n, r, gang):
         assert info.status == 0, info
         assert x.ranks == y.ranks
         assert _reldiff(x.cores[:], y.cores[:]) < 1e-8
+
+
+# the split Householder QR: less than a block of 16 columns, a block and one more,
+# two and one more, members without columns, 2304 rows (register blocks) and 2640
+# (LDS blocks)
+@pytest.mark.parametrize('d,n,r,gang', [(4, 6, 15, 2), (4, 6, 17, 3), (3, 40, 33, 5), (4, 5, 18, 32), (3, 72, 32, 2),
+                                        (3, 80, 33, 2)])
+def test_gang_rank_deficient_blocks(env, d, n, r, gang):
+    """alpha I x = b with b of rank 2 held at rank r: every panel is rank
+    deficient; the solution is b / alpha (bounds as above)."""
+    import scikit_tt_amd.solvers.sle as sle
+    print('case rank-deficient blocks d=%d n=%d r=%d gang=%d' % (d, n, r, gang), flush=True)
+    rng = np.random.default_rng(r)
+    A = W.shifted_operator(rng, d, n, sigma=0.0)
+    b = W.random_tt(rng, [n] * d, 2, scale=1.0 / np.sqrt(n))
+    ranks = [1] + [min(r, n ** min(k, d - k)) for k in range(1, d)] + [1]
+    x0 = W.random_tt(rng, [n] * d, ranks, scale=1.0 / np.sqrt(n))
+    (x,), (info,) = sle.als_gang([_tt(A)], [_tt(x0)], [_tt(b)], repeats=2, gang=gang, return_info=True)
+    assert info.status == 0, info
+    want = [c / float(d) if i == 0 else c for i, c in enumerate(b)]
+    assert _reldiff(x.cores[:], want) < 1e-9
+    for c in x.cores[1:]:  # right-orthonormal
+        m = np.asarray(c).reshape(c.shape[0], -1)
+        assert np.abs(m @ m.T - np.eye(c.shape[0])).max() < 1e-12
