@@ -1129,15 +1129,6 @@ __device__ int gang_hhqr_run(GangCtx& C, int m, int c) {
     hh_load_block<NB>(W, c, jb, rows, kb, Pn);
     __syncthreads();
     hh_block_factor<NB>(Pn, rows, kb, tau, G, dred, Yb);
-    if (C.g == 0) {
-      for (int i = threadIdx.x; i < rows; i += NT) {
-        double* dst = W + (long)(jb + i) * c + jb;
-#pragma unroll
-        for (int q = 0; q < NB; ++q)
-          if (q < kb) dst[q] = Pn[i * ld + q];
-      }
-      if (threadIdx.x < kb) D.tau[jb + threadIdx.x] = tau[threadIdx.x];
-    }
     hh_block_t<NB>(tau, G, kb, T);
     const int c2 = c - jb - kb;
     if (c2 > 0) {
@@ -1147,6 +1138,17 @@ __device__ int gang_hhqr_run(GangCtx& C, int m, int c) {
     }
     __syncthreads();
     if (!C.sync()) return -1;
+    // the factored block, once every member has loaded it
+    if (C.g == 0) {
+      for (int i = threadIdx.x; i < rows; i += NT) {
+        double* dst = W + (long)(jb + i) * c + jb;
+#pragma unroll
+        for (int q = 0; q < NB; ++q)
+          if (q < kb) dst[q] = Pn[i * ld + q];
+      }
+      if (threadIdx.x < kb) D.tau[jb + threadIdx.x] = tau[threadIdx.x];
+    }
+    __syncthreads();
   }
   // member 0: R, and W made the explicit V (unit diagonal, zeros above)
   if (C.g == 0) {
