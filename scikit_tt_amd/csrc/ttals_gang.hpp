@@ -566,7 +566,9 @@ __device__ __forceinline__ void gang_apply(const GangCtx& C, const GangLocal& o,
 // An iteration has a barrier for each of its two sums.  A third one completes
 // the direction where the matvec reads it from global memory; the on-chip
 // matvec reads the residual, complete by then, and adds the last direction's
-// first contraction, which it still holds.
+// first contraction, which it still holds (rounded like the direction itself;
+// errors against exact solutions over twelve -Laplacians, n = 9..24, ranks
+// 10..40, agree with the direct form's to 1 % in FP64, 15 % of 1e-14 in mixed).
 template <class T>
 __device__ TT_COLD int gang_cg(GangCtx& C, const GangLocal& o, const T* L, const T* A, const T* R, T* x, const T* f, T* r,
                        T* p, T* q, double tol, int maxit, int* iters, double* vfl) {
