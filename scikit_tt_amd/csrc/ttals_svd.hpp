@@ -1,12 +1,13 @@
 // One-sided (Hestenes) Jacobi SVD of a small matrix held in LDS.
 //
-// The arithmetic of wg_jacobi_svd (same pairing, rotations and convergence
-// test), reorganised: B and the accumulated rotations V sit in LDS by columns
-// (odd stride), a pair of columns takes L lanes (8 to 64) with its entries in
-// registers between the dot products and the rotation, and all pairs of a
-// round run at once.  A round is then bound by the LDS traffic of B and V and
-// one barrier instead of by global memory latency per column element, and the
-// final sort counts ranks in parallel instead of selecting on one thread.
+// The method of wg_jacobi_svd (same pairing, the same rotations up to rounding,
+// the same convergence test, here safe from underflow), reorganised: B and the
+// accumulated rotations V sit in LDS by columns (odd stride), a pair of columns
+// takes L lanes (8 to 64) with its entries in registers between the dot
+// products and the rotation, and all pairs of a round run at once.  A round is
+// then bound by the LDS traffic of B and V and one barrier instead of by global
+// memory latency per column element, and the final sort counts ranks in
+// parallel instead of selecting on one thread.
 // An 80 x 80 triangular factor of a rounding sweep: 5.5 ms in global memory
 // with one wave per pair, 0.8 ms here; one root and one division a rotation
 // then took a 64 x 64 one from 1.00 to 0.73 ms.
@@ -80,6 +81,14 @@ __device__ __forceinline__ void js_sweeps(TT_LDS double* Bl, TT_LDS double* Vl, 
         aii = lanes_sum(aii, L);
         ajj = lanes_sum(ajj, L);
         aij = lanes_sum(aij, L);
+        // the rotation depends on the ratios of the three sums alone: where a product of them could leave the range
+        // of a double (columns some 1e-60 below the largest), an exact power of two takes them near 1
+        if (fmin(aii, ajj) < 0x1p-400) {
+          const int e = -__builtin_amdgcn_frexp_exp(fmax(aii, ajj));
+          aii = ldexp(aii, e);
+          ajj = ldexp(ajj, e);
+          aij = ldexp(aij, e);
+        }
         if (fabs(aij) <= 1e-15 * sqrt(aii * ajj) || aij == 0.0) continue;
         // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)) for zeta = d / h: one root and one division
         const double d = ajj - aii, h = 2.0 * aij;
