@@ -46,18 +46,41 @@ __global__ __launch_bounds__(NT, TTALS_ALS_WAVES_PER_EU) void k_piece(PieceArgs 
 
 // TT core product (r1,m,n,r2) x (s1,n,p,s2) -> (r1*s1, m, p, r2*s2):
 // out[(i,k), mm, pp, (j,l)] = sum_nn A[i,mm,nn,j] X[k,nn,pp,l]
-//
-// Bound by the stores of `out` (2n flops for 8 bytes written).  A thread owns
-// one column (k, pp, l) of X -- or two neighbouring ones, V = dx2_t, s2 then
-// counting pairs -- with neighbouring threads on neighbouring l, and holds its
-// n entries in registers (NX >= n of them) while it walks the rows (i, mm) of
-// its blockIdx.y share: A's index is uniform over the wave (scalar loads),
-// every store of a wave is a run of consecutive l, and nothing is divided per
-// element (one element per thread cost six 64-bit divisions and two loads per
-// FMA).  NX = 0: n > 32, X read again from L1/L2 for every four values of j.
-// A rank-4 operator core times a (128, 16, 128) core, 33.5 MB out: 67 us one
-// element per thread, 19.3 us with one column, 14.4 us with two (2.3 TB/s of
-// stores, of which ~4 us are the launch).
+// in two forms; ttals_core_product says which takes a call.
+
+// One element per thread: six divisions and two loads per FMA, but as many
+// threads as there are elements and stores that are always consecutive.  I:
+// the index type (unsigned below 2^31 elements).
+template <class I>
+__global__ __launch_bounds__(256) void k_core_product_elem(int r1, int m, int n, int r2, int s1, int p, int s2,
+                                                           const double* __restrict__ A, const double* __restrict__ X,
+                                                           double* __restrict__ out) {
+  const I total = (I)r1 * s1 * m * p * r2 * s2;
+  for (I e = blockIdx.x * (I)blockDim.x + threadIdx.x; e < total; e += (I)gridDim.x * blockDim.x) {
+    I t = e;
+    const I l = t % s2; t /= s2;
+    const I j = t % r2; t /= r2;
+    const I pp = t % p; t /= p;
+    const I mm = t % m; t /= m;
+    const I k = t % s1, i = t / s1;
+    const double* ap = A + (long)(i * m + mm) * n * r2 + j;
+    const double* xp = X + ((long)k * n * p + pp) * s2 + l;
+    double s = 0.0;
+    for (int q = 0; q < n; ++q) s += ap[(long)q * r2] * xp[(long)q * p * s2];
+    out[e] = s;
+  }
+}
+
+// By columns.  Bound by the stores of `out` (2n flops for 8 bytes written).  A
+// thread owns one column (k, pp, l) of X -- or two neighbouring ones, V =
+// dx2_t, s2 then counting pairs -- with neighbouring threads on neighbouring l,
+// and holds its n entries in registers (NX >= n of them) while it walks the
+// rows (i, mm) of its blockIdx.y share: A's index is uniform over the wave
+// (scalar loads), every store of a wave is a run of consecutive l, and nothing
+// is divided per element.  NX = 0: n > 32, X read again from L1/L2 for every
+// four values of j.  A rank-4 operator core times a (128, 16, 128) core,
+// 33.5 MB out: 67 us one element per thread, 19.3 us with one column, 14.4 us
+// with two (2.3 TB/s of stores, of which ~4 us are the launch).
 template <int NX, class V>
 __global__ __launch_bounds__(256) void k_core_product(int r1, int m, int n, int r2, int s1, int p, int s2,
                                                       const double* __restrict__ A, const V* __restrict__ X,
@@ -2230,11 +2253,28 @@ int ttals_core_product(void* stream, int r1, int m, int n, int r2, int s1, int p
   const bool two = s2 % 2 == 0 && ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
   const int w = two ? s2 / 2 : s2;
   const long cols = (long)s1 * p * w, bx = (cols + 255) / 256, rows = (long)r1 * m;
-  if (bx > 0x7fffffffL || rows > 0x7fffffffL) return TTALS_E_ARG;
   // rows are split until the launch has about 1024 workgroups (four waves per
   // SIMD): each share reads its columns of X again.  The (128, 16, 128) core
   // above: 30.0, 17.2, 14.4, 16.9 us at 256, 512, 1024, 2048 workgroups
   const unsigned by = (unsigned)std::max<long>(1, std::min<long>(std::min<long>(rows, 65535), (1024 + bx - 1) / bx));
+  // The column form's threads each work through a chain of q's and j's (about
+  // 24 ns a term, over the rows and j's of a share; a j outside the groups of
+  // four counts twice), which only enough columns hide; the element form costs
+  // about half a ps per term of the whole product and 50 ns per q.  The cheaper
+  // of the two by that estimate: over 560 shapes, ranks up to 300, within 1 %
+  // of the better form on average.  A (128, 16, 16, 128) operator core times a
+  // (1, 16, 1, 1) core: 210 us by columns, 6.9 us by elements; (1, 1, 64, 200)
+  // times (1, 64, 1, 200), an inner product's first core: 364 and 9.6 us; a
+  // 1000 x 1000 matrix times a vector: 67 and 131 us (and the header of
+  // k_core_product).  Launches past the grid's limits by elements too.
+  const long total = rows * s1 * p * ((long)r2 * s2);
+  const double chain = (double)((rows + by - 1) / by) * n * (4 * (r2 / 4) + 2 * (r2 % 4));
+  if (chain * 48e3 > std::max((n + 2.0) * (double)total, 1e5 * n) || bx >= (1L << 24) || rows > 0x7fffffffL) {
+    const unsigned blocks = (unsigned)std::min<long>((total + 255) / 256, 65536);
+    hipLaunchKernelGGL(total < (1L << 31) ? k_core_product_elem<unsigned> : k_core_product_elem<unsigned long>,
+                       dim3(blocks), dim3(256), 0, (hipStream_t)stream, r1, m, n, r2, s1, p, s2, A, X, out);
+    return hipGetLastError() == hipSuccess ? 0 : TTALS_E_HIP;
+  }
   const dim3 grid((unsigned)bx, by);
   auto go = [&](auto nx) {
     constexpr int NX = decltype(nx)::value;
