@@ -36,14 +36,29 @@ __device__ __forceinline__ double lanes_sum(double v, int L) {
   return v;
 }
 
+// Factors of up to JS_ONE columns and rows are one wave's work: the barriers of
+// eight waves cost more than the rotations (truncated_svd of an 8 x 8 matrix:
+// 108 us with eight waves, 80 us with one, the same bits).
+constexpr int JS_ONE = 16;
+// a barrier of the working threads: the workgroup, or (ONE) the first wave alone
+template <bool ONE>
+__device__ __forceinline__ void js_sync() {
+  if constexpr (ONE) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
 // Sweeps of rotations over all column pairs of Bl (k columns, c rows, ld lb)
 // and Vl (k rows, ld lv) until a sweep rotates nothing (at most 60): RM entries
 // of a column per lane, L lanes per pair (RM * L >= c, k).
-template <int RM>
+template <int RM, bool ONE>
 __device__ __forceinline__ void js_sweeps(TT_LDS double* Bl, TT_LDS double* Vl, int c, int k, int lb, int lv, int L,
                                           int* s_rot) {
   const int kk = (k & 1) ? k + 1 : k, pairs = kk / 2, mod = kk - 1;
-  const int l = threadIdx.x & (L - 1), g = threadIdx.x / L, ng = NT / L;
+  const int l = threadIdx.x & (L - 1), g = threadIdx.x / L, ng = (ONE ? 64 : NT) / L;
   for (int sweep = 0; sweep < 60; ++sweep) {
     const int flag = sweep & 1;
     for (int round = 0; round < mod; ++round) {
@@ -82,14 +97,16 @@ __device__ __forceinline__ void js_sweeps(TT_LDS double* Bl, TT_LDS double* Vl, 
         ajj = lanes_sum(ajj, L);
         aij = lanes_sum(aij, L);
         // the rotation depends on the ratios of the three sums alone: where a product of them could leave the range
-        // of a double (columns some 1e-60 below the largest), an exact power of two takes them near 1
-        if (fmin(aii, ajj) < 0x1p-400) {
+        // of a double (columns some 1e-70 below the largest), an exact power of two takes them near 1
+        double prod = aii * ajj;
+        if (__builtin_expect(__any(prod < 0x1p-900), 0)) {
           const int e = -__builtin_amdgcn_frexp_exp(fmax(aii, ajj));
           aii = ldexp(aii, e);
           ajj = ldexp(ajj, e);
           aij = ldexp(aij, e);
+          prod = aii * ajj;
         }
-        if (fabs(aij) <= 1e-15 * sqrt(aii * ajj) || aij == 0.0) continue;
+        if (fabs(aij) <= 1e-15 * sqrt(prod) || aij == 0.0) continue;
         // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)) for zeta = d / h: one root and one division
         const double d = ajj - aii, h = 2.0 * aij;
         const double t = (d >= 0.0 ? h : -h) / (fabs(d) + sqrt(fma(d, d, h * h)));
@@ -108,11 +125,11 @@ __device__ __forceinline__ void js_sweeps(TT_LDS double* Bl, TT_LDS double* Vl, 
         }
         if (l == 0) s_rot[flag] = 1;
       }
-      __syncthreads();
+      js_sync<ONE>();
     }
     const int rot = s_rot[flag];
     if (threadIdx.x == 0) s_rot[flag ^ 1] = 0;
-    __syncthreads();
+    js_sync<ONE>();
     if (rot == 0) break;
   }
 }
@@ -121,46 +138,57 @@ __device__ __forceinline__ void js_sweeps(TT_LDS double* Bl, TT_LDS double* Vl, 
 // x k, row-major, global) the rotations; sig the column norms, perm the
 // columns by decreasing norm.  lds: js_doubles(c, k).  B is scaled by a power
 // of two (exactly) while it is worked on, so that the squares of its norms
-// neither overflow nor vanish.  Starts and ends with a barrier.
-__device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, int* perm, double* lds_) {
+// neither overflow nor vanish.  The work of wg_jacobi_lds between its barriers,
+// by the whole workgroup or (ONE) by its first wave.
+template <bool ONE>
+__device__ __attribute__((noinline)) void js_run(double* B, int c_, int k_, double* V, double* sig, int* perm,
+                                                 double* lds_) {
+  constexpr int TH = ONE ? 64 : NT;
   __shared__ int s_rot[2];
   __shared__ double s_mx[NWAVE];
+  const int c = uni(c_), k = uni(k_);
   TT_LDS double* Bl = (TT_LDS double*)lds_;
   const int lb = c | 1, lv = k | 1;
   TT_LDS double* Vl = Bl + k * lb;
   TT_LDS double* sg = Vl + k * lv;
-  __syncthreads();
-  double mx = 0.0;
-  for (int e = threadIdx.x; e < c * k; e += NT) mx = fmax(mx, fabs(B[e]));
+  // the first TH entries stay in registers for the scaled copy below (all of a small factor)
+  const int n = c * k;
+  const double first = threadIdx.x < n ? B[threadIdx.x] : 0.0;
+  double mx = fabs(first);
+  for (int e = threadIdx.x + TH; e < n; e += TH) mx = fmax(mx, fabs(B[e]));
   mx = wave_max(mx);
   if ((threadIdx.x & 63) == 0) s_mx[threadIdx.x >> 6] = mx;
   if (threadIdx.x < 2) s_rot[threadIdx.x] = 0;
-  __syncthreads();
+  for (int e = threadIdx.x; e < k * lv; e += TH) {
+    const int j = e / lv, i = e - j * lv;
+    Vl[e] = i == j ? 1.0 : 0.0;
+  }
+  js_sync<ONE>();
 #pragma unroll
-  for (int q = 0; q < NWAVE; ++q) mx = fmax(mx, s_mx[q]);
+  for (int q = 0; q < (ONE ? 1 : NWAVE); ++q) mx = fmax(mx, s_mx[q]);
   const int ex = (mx > 0.0 && isfinite(mx)) ? -ilogb(mx) : 0;  // applied in two halves: 2^ex itself may overflow
   const double up0 = ldexp(1.0, ex / 2), up1 = ldexp(1.0, ex - ex / 2);
   const double dn0 = ldexp(1.0, -(ex / 2)), dn1 = ldexp(1.0, ex / 2 - ex);
-  for (int e = threadIdx.x; e < c * k; e += NT) {
+  for (int e = threadIdx.x; e < n; e += TH) {
     const int i = e / k, j = e - i * k;
-    Bl[j * lb + i] = B[e] * up0 * up1;
-  }
-  for (int e = threadIdx.x; e < k * lv; e += NT) {
-    const int j = e / lv, i = e - j * lv;
-    Vl[e] = i == j ? 1.0 : 0.0;
+    Bl[j * lb + i] = (e < TH ? first : B[e]) * up0 * up1;
   }
   const int rows = c > k ? c : k, pairs = (k + 1) / 2;
   int L = 8;
   while (rows > L * JS_ROWS) L <<= 1;
-  while (L < 64 && 2 * L * pairs <= NT) L <<= 1;
-  L = __builtin_amdgcn_readfirstlane(L);
-  __syncthreads();
-  if (rows <= 2 * L) js_sweeps<2>(Bl, Vl, c, k, lb, lv, L, s_rot);
-  else if (rows <= 4 * L) js_sweeps<4>(Bl, Vl, c, k, lb, lv, L, s_rot);
-  else if (rows <= 8 * L) js_sweeps<8>(Bl, Vl, c, k, lb, lv, L, s_rot);
-  else js_sweeps<JS_ROWS>(Bl, Vl, c, k, lb, lv, L, s_rot);
+  while (L < 64 && 2 * L * pairs <= TH) L <<= 1;
+  L = ONE ? JS_ONE : __builtin_amdgcn_readfirstlane(L);  // ONE: an entry per lane, the sums of the other form
+  js_sync<ONE>();
+  if constexpr (ONE) {
+    js_sweeps<1, true>(Bl, Vl, c, k, lb, lv, L, s_rot);
+  } else {
+    if (rows <= 2 * L) js_sweeps<2, false>(Bl, Vl, c, k, lb, lv, L, s_rot);
+    else if (rows <= 4 * L) js_sweeps<4, false>(Bl, Vl, c, k, lb, lv, L, s_rot);
+    else if (rows <= 8 * L) js_sweeps<8, false>(Bl, Vl, c, k, lb, lv, L, s_rot);
+    else js_sweeps<JS_ROWS, false>(Bl, Vl, c, k, lb, lv, L, s_rot);
+  }
   // column norms (a non-finite one sorts first) and ranks by decreasing norm
-  for (int j = threadIdx.x; j < k; j += NT) {
+  for (int j = threadIdx.x; j < k; j += TH) {
     double s0 = 0.0, s1 = 0.0;
     for (int r = 0; r + 1 < c; r += 2) {
       s0 = fma(Bl[j * lb + r], Bl[j * lb + r], s0);
@@ -171,21 +199,28 @@ __device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, i
     sig[j] = s * dn0 * dn1;
     sg[j] = s == s ? s : INFINITY;
   }
-  __syncthreads();
-  for (int j = threadIdx.x; j < k; j += NT) {
+  js_sync<ONE>();
+  for (int j = threadIdx.x; j < k; j += TH) {
     const double s = sg[j];
     int rank = 0;
     for (int q = 0; q < k; ++q) rank += (sg[q] > s || (sg[q] == s && q < j)) ? 1 : 0;
     perm[rank] = j;
   }
-  for (int e = threadIdx.x; e < c * k; e += NT) {
+  for (int e = threadIdx.x; e < c * k; e += TH) {
     const int i = e / k, j = e - i * k;
     B[e] = Bl[j * lb + i] * dn0 * dn1;
   }
-  for (int e = threadIdx.x; e < k * k; e += NT) {
+  for (int e = threadIdx.x; e < k * k; e += TH) {
     const int i = e / k, j = e - i * k;
     V[e] = Vl[j * lv + i];
   }
+}
+
+// Starts and ends with a barrier.
+__device__ void wg_jacobi_lds(double* B, int c, int k, double* V, double* sig, int* perm, double* lds) {
+  __syncthreads();
+  if (c > JS_ONE || k > JS_ONE) js_run<false>(B, c, k, V, sig, perm, lds);
+  else if (threadIdx.x < 64) js_run<true>(B, c, k, V, sig, perm, lds);
   __syncthreads();
 }
 

@@ -6,6 +6,7 @@
 // the QR, and the QR's block lives in the registers of all eight waves), so
 // the building blocks are compiled for 512 threads here.
 #define TTALS_NT 512
+#define TTALS_QR_IEEE
 #include "ttals_tt.hpp"
 
 #include "ttals_dev.hpp"
@@ -41,24 +42,66 @@ __device__ int count_kept(const double* sig, const int* perm, int k, double thr,
   return (int)wg_sum(n, red);
 }
 
+// Panels that the register QR (wg_qr_small) takes, copied to LDS, instead of the
+// blocks: there a block of 16 columns costs more than the panel (rounding of a
+// train of order 4, n = 2, ranks 2: 105 us with blocks, 93 us so; its residual
+// norm 181 and 160 us).
+__device__ __forceinline__ bool qr_in_lds(int m, int c) { return (m <= 32 && c <= 32) || (m <= 64 && c <= 16); }
+static_assert(8 * (4 * 1024 + 64) <= TT_LDS_BYTES, "panel, Q, R and tau of the register QR");
+// R on and above W's diagonal, the reflectors below it; Q into Qm where wanted.
+__device__ void qr_small(double* W, int m, int c, double* Qm, const TtLDS& S) {
+  const int k = m < c ? m : c;
+  double *w = S.gemm, *q = w + 1024, *r = q + 1024, *t = r + 1024;
+  __syncthreads();
+  for (int e = threadIdx.x; e < m * c; e += NT) w[e] = W[e];
+  __syncthreads();
+  wg_qr_small(w, m, c, t, q, r);
+  for (int e = threadIdx.x; e < m * c; e += NT) W[e] = w[e];
+  if (Qm)
+    for (int e = threadIdx.x; e < m * k; e += NT) Qm[e] = q[e];
+  __syncthreads();
+}
+// A column, or two of some hundred rows: the column sweep (100 x 1: 50 us a
+// truncated sweep, 55 us with a block).
+__device__ __forceinline__ bool qr_by_columns(int m, int c) { return m <= 256 && (c == 1 || (c == 2 && m > 64)); }
+
 // R of the QR of the panel W (m x c, row-major, overwritten): in the top rows
 // of the returned matrix (row stride c).  Panels of more columns than half
 // the rows a block holds take the column sweep.
 __device__ const double* qr_r(double* W, int m, int c, double* tau, const TtLDS& S, double* red) {
-  if ((m <= HQ_ROWS_MAX || 2 * c <= HQ_ROWS_MAX) && hq_fits(m, c)) return wg_hqr_r(W, m, c, c, S.qr);
+  const bool by_columns = qr_by_columns(m, c);
+  if (!by_columns && qr_in_lds(m, c)) {
+    qr_small(W, m, c, nullptr, S);
+    return W;
+  }
+  if (!by_columns && (m <= HQ_ROWS_MAX || 2 * c <= HQ_ROWS_MAX) && hq_fits(m, c))
+    return wg_hqr_r(W, m, c, c, S.qr);
   wg_householder(W, m, c, tau, red);
   return W;
 }
 
 // The same with the reflectors left in W and the explicit Q (m x min(m, c))
 // in Qm; the column sweep for panels taller than a block holds.
-__device__ void qr_rq(double* W, int m, int c, double* tau, double* Tg, double* Qm, const TtLDS& S, double* red) {
+__device__ void qr_rq_blocks(double* W, int m, int c, double* tau, double* Tg, double* Qm, const TtLDS& S,
+                             double* red) {
   if (m <= HQ_ROWS_MAX && hq_fits(m, c)) {
     wg_hqr(W, m, c, c, Tg, S.qr);
     wg_hqr_form_q(W, m, c, c, Tg, Qm, S.qr);
   } else {
     wg_householder(W, m, c, tau, red);
     wg_form_q(W, m, c, tau, Qm);
+  }
+}
+
+// ... with the forms for small panels.
+__device__ void qr_rq(double* W, int m, int c, double* tau, double* Tg, double* Qm, const TtLDS& S, double* red) {
+  if (qr_by_columns(m, c)) {
+    wg_householder(W, m, c, tau, red);
+    wg_form_q(W, m, c, tau, Qm);
+  } else if (qr_in_lds(m, c)) {
+    qr_small(W, m, c, Qm, S);
+  } else {
+    qr_rq_blocks(W, m, c, tau, Tg, Qm, S, red);
   }
 }
 
@@ -282,7 +325,10 @@ __global__ __launch_bounds__(NT) void k_svd_trunc(SvdArgs A) {
     A.W[e] = tall ? A.Y[e] : A.Y[(long)j * A.c + i];
   }
   __syncthreads();
-  qr_rq(A.W, mt, ct, A.tau, A.Tg, A.Qm, S, red);
+  // the small panels' forms from two columns on would save some 4 us a call, but a threshold near rounding then cuts
+  // elsewhere (the two-site solver's ranks at 1e-14)
+  if (ct == 1) qr_rq(A.W, mt, ct, A.tau, A.Tg, A.Qm, S, red);
+  else qr_rq_blocks(A.W, mt, ct, A.tau, A.Tg, A.Qm, S, red);
   // B = R^T (ct x ct)
   for (long e = threadIdx.x; e < (long)ct * ct; e += NT) {
     const int i = (int)(e / ct), j = (int)(e % ct);
