@@ -30,3 +30,21 @@ def load_golden(name):
 @pytest.fixture
 def golden():
     return load_golden
+
+
+@pytest.fixture(scope='module', autouse=True)
+def contexts_of_the_module():
+    """Every module gets shared engine contexts of its own: what a test sets on
+    one (an arena of its choice switches the automatic choice of kernels off
+    for good) ends with the module."""
+    from scikit_tt_amd import _lib
+    saved = dict(_lib._ctx)
+    _lib._ctx.clear()
+    yield
+    if _lib._ctx:
+        import torch
+        torch.cuda.synchronize()
+        for ctx in _lib._ctx.values():
+            _lib.load().ttals_ctx_destroy(ctx)
+    _lib._ctx.clear()
+    _lib._ctx.update(saved)
