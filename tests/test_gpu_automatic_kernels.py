@@ -138,3 +138,49 @@ def test_one_schedule(two):
     for s, (d, n, r) in enumerate(sizes):
         same = all(torch.equal(c, e) for c, e in zip(here[s].device_cores, there[s].device_cores))
         assert same == (n * r * r < 10240), (s, same)
+
+
+def _time_us(lib, entry, ctx, args):
+    best = float('inf')
+    for _ in range(5):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(20):
+            assert getattr(lib, entry)(ctx, None, *args) == 0
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 50.0)
+    return best
+
+
+@pytest.mark.parametrize('entry,dims', [('ttals_stack_left_rhs', (32, 4, 64, 1, 4)),
+                                        ('ttals_stack_left_rhs', (16, 3, 16, 1, 48)),
+                                        ('ttals_stack_left_op', (16, 2, 64, 1, 4)),
+                                        ('ttals_stack_right_op', (3, 1, 64, 3, 16)),
+                                        ('ttals_stack_right_rhs', (32, 4, 64, 1, 4)),
+                                        ('ttals_micro_rhs', (16, 4, 64, 4, 2))])
+def test_global_memory_pieces_take_the_faster_kernel(two, entry, dims):
+    """The same result as on the four-wave kernel, and no slower (148 and
+    182 us for the first one when eight waves took every piece)."""
+    lib, auto, pinned = two
+    a, p, n, q, b = dims
+    gen = torch.Generator(device='cuda').manual_seed(sum(dims))
+    op = entry.endswith('_op')
+    left = edges._randn(gen, *((a, p, a) if op else (p, a)))
+    right = edges._randn(gen, *((b, q, b) if op else (q, b)))
+    core = edges._randn(gen, p, n, n, q) if op else edges._randn(gen, p, n, q)
+    x = edges._randn(gen, a, n, b)
+    outs = [torch.full((a * n * b if 'micro' in entry else (b * q * b if 'left' in entry else a * p * a) if op else
+                        (q * b if 'left' in entry else p * a),), float('nan'), dtype=torch.float64, device='cuda')
+            for _ in range(2)]
+    us = []
+    for ctx, out in zip((auto, pinned), outs):
+        first = [left, core, right, out] if 'micro' in entry else \
+            [left if 'left' in entry else right, core, x, out]
+        us.append(_time_us(lib, entry, ctx, (a, p, n, q, b, *map(_ptr, first))))
+    print('  %.1f us, four waves %.1f us' % tuple(us), flush=True)
+    # sums of K N(0, 1) products: K eps times the sum of the magnitudes, which exceeds the largest sum by less than
+    # the number of its terms' square root
+    bound = 4 * (a + p * n + a * n + n * q + n * b) * EPS * float(outs[1].abs().max()) * a * b * n * p * q
+    assert float((outs[0] - outs[1]).abs().max()) <= bound
+    assert us[0] <= 1.12 * us[1]
