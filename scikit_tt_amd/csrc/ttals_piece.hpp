@@ -166,8 +166,10 @@ __device__ __forceinline__ void piece_block(const PieceArgs& A, double* dyn_lds,
     }
     case P_QR: {
       // m = a, c = b; input x (m x c); out = Q (m x k); v = R (k x c); t1 = work
-      // (W, then tau, then (c + 16) * 16 for the blocked QR's T); the
-      // engine's choice of method for a global-memory panel (qr_factor)
+      // (W, then tau, then (c + 16) * 16 for the blocked QR's T).  The forms the
+      // engine keeps for panels of up to 64 x 64 and for those of more rows than
+      // wg_hqr holds; its register-blocked QR would be a second caller of wg_hqr
+      // in k_als's translation unit, which costs k_als 28 more spilled registers.
       const int m = A.a, c = A.b;
       double* W = A.t1;
       for (long e = threadIdx.x; e < (long)m * c; e += NT) W[e] = A.x[e];
