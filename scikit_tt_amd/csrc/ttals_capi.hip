@@ -1293,49 +1293,11 @@ int piece_scratch(ttals_ctx* c, long t, long N, double** t1, double** t2, double
   return 0;
 }
 
-// K-steps (of 16) of a global-memory GEMM: output tiles of 64 x 64 with four
-// waves, 128 x 64 with eight (the longer side of the output along the longer
-// side of the tile).
-long gemm_steps(long M, long N, long K, bool wide) {
-  if (wide && M <= 64 && N > M) std::swap(M, N);
-  return ((M + (wide ? 127 : 63)) / (wide ? 128 : 64)) * ((N + 63) / 64) * ((K + 15) / 16);
-}
-
-// Does a piece that stays in global memory gain from eight waves?  A K-step of
-// one tile costs 1.25 us with four waves and 1.5 us with eight, whose launch
-// costs 0.8 us more: eight waves pay where the output has several tiles (right
-// interface of a rhs of rank 4, a = 32, n = 64, b = 1: 60.6 -> 40.4 us), not
-// where one tile walks a long K (its left interface: 148 and 182 us).
-bool piece_steps_wide(const PieceArgs& a) {
-  const long A = a.a, P = a.P, n = a.n, Q = a.Q, b = a.b;
-  long s[2];
-  for (int w = 0; w < 2; ++w) {
-    auto g = [&](long M, long N, long K) { return gemm_steps(M, N, K, w == 1); };
-    switch (a.op) {
-      case P_LEFT_OP: s[w] = g(P * A, n * b, A) + g(A * b, n * Q, P * n) + g(b * Q, b, A * n); break;
-      case P_RIGHT_OP: s[w] = g(A * n, b * Q, b) + g(A * b, P * n, n * Q) + g(A, P * A, n * b); break;
-      case P_LEFT_RHS: s[w] = g(A, n * Q, P) + g(Q, b, A * n); break;
-      case P_RIGHT_RHS: s[w] = g(A * n, Q, b) + g(P, A, n * Q); break;
-      default: s[w] = g(A, n * Q, P) + g(A * n, b, Q); break;  // P_MICRO_RHS
-    }
-  }
-  return 6 * s[1] + 3 < 5 * s[0];
-}
-
-// LDS of a stack update on chip (as piece_block counts it).
-long piece_stack_need(const PieceArgs& a) {
-  const bool left = a.op == P_LEFT_OP;
-  const int al = left ? a.a : a.b, Pl = left ? a.P : a.Q, Ql = left ? a.Q : a.P, bl = left ? a.b : a.a;
-  return (long)al * Pl * al + (long)a.a * a.n * a.b + (long)a.P * a.n * a.n * a.Q + ds_t1_size(al, Pl, a.n, bl) +
-         ds_t2_size(al, a.n, Ql, bl) + (long)bl * Ql * bl;
-}
-
 int launch_piece(ttals_ctx* c, hipStream_t st, PieceArgs& a) {
   a.arena = c->arena;
   a.mvar = c->matvec_variant;
   // local problems off k_als's arena on eight waves with the CU's LDS (an
-  // arena the caller chose, and panels, stay here); of the pieces that work in
-  // global memory even there, those that eight waves shorten
+  // arena the caller chose, and panels, stay here)
   if (a.op != P_QR && !c->arena_set &&
       arena_need_onchip(a.a, a.P, a.n, a.Q, a.b, a.op == P_EIG ? 3 : 5, a.mvar) > c->arena) {
     if (c->arena_piece == 0) {
@@ -1345,14 +1307,9 @@ int launch_piece(ttals_ctx* c, hipStream_t st, PieceArgs& a) {
       HIPCHK(c, piece_wide_static_lds(&stat));
       c->arena_piece = std::max(c->arena, ((long)max_lds - (long)stat - 1024) / 8);
     }
-    const bool stack = a.op == P_LEFT_OP || a.op == P_RIGHT_OP;
-    const bool rhs = a.op == P_LEFT_RHS || a.op == P_RIGHT_RHS || a.op == P_MICRO_RHS;
-    const bool global = rhs || (stack && piece_stack_need(a) > c->arena_piece);
-    if (!global || piece_steps_wide(a)) {
-      a.arena = c->arena_piece;
-      HIPCHK(c, piece_wide_launch((size_t)a.arena * 8, st, a));
-      return 0;
-    }
+    a.arena = c->arena_piece;
+    HIPCHK(c, piece_wide_launch((size_t)a.arena * 8, st, a));
+    return 0;
   }
   hipLaunchKernelGGL(k_piece, dim3(1), dim3(NT), (size_t)a.arena * 8, st, a);
   HIPCHK(c, hipGetLastError());

@@ -290,6 +290,14 @@ __device__ __forceinline__ void wg_fill(T* y, T v, int n) {
 // a 32 x 32 quadrant per wave.
 
 constexpr int GBM = NT / 4, GBN = 64, GBK = 16;
+// Eight waves: those whose quadrant of a tile lies past the output's edge leave
+// LDS and matrix cores to the others (half of them do nothing else in an output
+// of up to 64 rows).  Same bits; a two-member gang on a system of order 4,
+// n = 6, ranks 6: 1781 us without, 1655 us with; a two-site sweep, n = 8, ranks
+// 8: 11.4 and 10.6 ms; residual norm of a train with modes 500: 9.0 and 7.9 ms.
+// Where the outputs fill the tiles the test costs up to 1 %.
+constexpr bool GEMM_EDGE = NT == 512;
+
 constexpr int GEMM_LDS_DOUBLES = GBK * (GBM + 1) + GBK * (GBN + 1);
 
 // i -> (i / div) * hi + (i % div) * lo for 0 <= i < 2^22 with an FP32
@@ -410,15 +418,17 @@ __device__ __forceinline__ void wg_gemm_mf(int M, int N, int K, CView<T> A, CVie
   __syncthreads();
   for (int s = 0; s < steps; ++s) {
     if (s + 1 < steps) load(ra, rb);
+    if (!GEMM_EDGE || (cm0 + wm < M && cn0 + wn < N)) {
 #pragma unroll
-    for (int q = 0; q < GBK / 4; ++q) {
-      const int kr = (4 * q + lk);
-      const T a0 = As[kr * (GBM + 1) + wm + li], a1 = As[kr * (GBM + 1) + wm + 16 + li];
-      const T b0 = Bs[kr * (GBN + 1) + wn + li], b1 = Bs[kr * (GBN + 1) + wn + 16 + li];
-      acc[0][0] = mfma16x16x4(a0, b0, acc[0][0]);
-      acc[0][1] = mfma16x16x4(a0, b1, acc[0][1]);
-      acc[1][0] = mfma16x16x4(a1, b0, acc[1][0]);
-      acc[1][1] = mfma16x16x4(a1, b1, acc[1][1]);
+      for (int q = 0; q < GBK / 4; ++q) {
+        const int kr = (4 * q + lk);
+        const T a0 = As[kr * (GBM + 1) + wm + li], a1 = As[kr * (GBM + 1) + wm + 16 + li];
+        const T b0 = Bs[kr * (GBN + 1) + wn + li], b1 = Bs[kr * (GBN + 1) + wn + 16 + li];
+        acc[0][0] = mfma16x16x4(a0, b0, acc[0][0]);
+        acc[0][1] = mfma16x16x4(a0, b1, acc[0][1]);
+        acc[1][0] = mfma16x16x4(a1, b0, acc[1][0]);
+        acc[1][1] = mfma16x16x4(a1, b1, acc[1][1]);
+      }
     }
     ckk += GBK;
     if (ckk >= K) {
