@@ -1428,7 +1428,8 @@ __device__ __forceinline__ double qr_div(double a, double b) { return a / b; }
 #else
 __device__ __forceinline__ double qr_div(double a, double b) { return a * rcp_nr(b); }
 #endif
-template <int R, int C>
+// WITH_Q false: W and tau alone.
+template <int R, int C, bool WITH_Q = true>
 __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, double* Rm) {
   const int l16 = threadIdx.x & 15, r = threadIdx.x >> 4;  // lane in row, DPP row
   const int k = m < c ? m : c;
@@ -1512,6 +1513,7 @@ __device__ void wg_qr_small_t(double* W, int m, int c, double* tau, double* Qm, 
       if (jj >= k && jj < c && i < m) W[i * c + jj] = a[q][u];
     }
   __syncthreads();
+  if constexpr (!WITH_Q) return;
   const float ic = 1.0f / (float)c;
   for (int e = threadIdx.x; e < k * c; e += NT) {
     const int i = fquot(e, ic), jj = e - i * c;

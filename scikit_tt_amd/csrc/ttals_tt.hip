@@ -48,16 +48,22 @@ __device__ int count_kept(const double* sig, const int* perm, int k, double thr,
 // norm 181 and 160 us).
 __device__ __forceinline__ bool qr_in_lds(int m, int c) { return (m <= 32 && c <= 32) || (m <= 64 && c <= 16); }
 static_assert(8 * (4 * 1024 + 64) <= TT_LDS_BYTES, "panel, Q, R and tau of the register QR");
-// R on and above W's diagonal, the reflectors below it; Q into Qm where wanted.
+// R on and above W's diagonal, the reflectors below it; Q into Qm.
+template <bool WITH_Q>
 __device__ void qr_small(double* W, int m, int c, double* Qm, const TtLDS& S) {
   const int k = m < c ? m : c;
   double *w = S.gemm, *q = w + 1024, *r = q + 1024, *t = r + 1024;
   __syncthreads();
   for (int e = threadIdx.x; e < m * c; e += NT) w[e] = W[e];
   __syncthreads();
-  wg_qr_small(w, m, c, t, q, r);
+  if constexpr (WITH_Q) {
+    wg_qr_small(w, m, c, t, q, r);
+  } else {  // m <= 32, c <= 16
+    if (m <= 16) wg_qr_small_t<1, 1, false>(w, m, c, t, q, r);
+    else wg_qr_small_t<2, 1, false>(w, m, c, t, q, r);
+  }
   for (int e = threadIdx.x; e < m * c; e += NT) W[e] = w[e];
-  if (Qm)
+  if constexpr (WITH_Q)
     for (int e = threadIdx.x; e < m * k; e += NT) Qm[e] = q[e];
   __syncthreads();
 }
@@ -67,12 +73,17 @@ __device__ __forceinline__ bool qr_by_columns(int m, int c) { return m <= 256 &&
 
 // R of the QR of the panel W (m x c, row-major, overwritten): in the top rows
 // of the returned matrix (row stride c).  Panels of more columns than half
-// the rows a block holds take the column sweep.
+// the rows a block holds take the column sweep.  SMALL: the register QR up to
+// 32 x 16 (alone, it gains nothing on R: the norm of a train of order 4,
+// n = 4, ranks 4 takes 53 us either way).
+template <bool SMALL>
 __device__ const double* qr_r(double* W, int m, int c, double* tau, const TtLDS& S, double* red) {
   const bool by_columns = qr_by_columns(m, c);
-  if (!by_columns && qr_in_lds(m, c)) {
-    qr_small(W, m, c, nullptr, S);
-    return W;
+  if constexpr (SMALL) {
+    if (!by_columns && m <= 32 && c <= 16) {
+      qr_small<false>(W, m, c, nullptr, S);
+      return W;
+    }
   }
   if (!by_columns && (m <= HQ_ROWS_MAX || 2 * c <= HQ_ROWS_MAX) && hq_fits(m, c))
     return wg_hqr_r(W, m, c, c, S.qr);
@@ -99,7 +110,7 @@ __device__ void qr_rq(double* W, int m, int c, double* tau, double* Tg, double* 
     wg_householder(W, m, c, tau, red);
     wg_form_q(W, m, c, tau, Qm);
   } else if (qr_in_lds(m, c)) {
-    qr_small(W, m, c, Qm, S);
+    qr_small<true>(W, m, c, Qm, S);
   } else {
     qr_rq_blocks(W, m, c, tau, Tg, Qm, S, red);
   }
@@ -162,7 +173,7 @@ __device__ double resid_sweep(const ResidDesc& D, bool with_ax, const TtLDS& S, 
       __syncthreads();
       return wg_nrm2(v, mk, red);
     }
-    const double* R = qr_r(D.W, mk, rho, D.tau, S, red);
+    const double* R = qr_r<true>(D.W, mk, rho, D.tau, S, red);
     const int kk = mk < rho ? mk : rho;
     for (int e = threadIdx.x; e < kk * rho; e += NT) {
       const int r = e / rho, c = e - r * rho;
@@ -204,7 +215,7 @@ __global__ __launch_bounds__(NT) void k_tt_norm(NormArgs A) {
       A.W[e] = ci[(long)jj * m + ii];
     }
     __syncthreads();
-    const double* R = qr_r(A.W, m, c, A.tau, S, red);
+    const double* R = qr_r<false>(A.W, m, c, A.tau, S, red);
     const int k = m < c ? m : c;
     for (long e = threadIdx.x; e < (long)k * c; e += NT) {
       const int ii = (int)(e / c), jj = (int)(e % c);
