@@ -165,8 +165,10 @@ int ttals_wait(ttals_ctx* ctx, ttals_result* res);
 /* Size of the on-chip (LDS) arena in KB, 0..61 (default 61): local
  * problems whose operator and working vectors fit run LDS-resident on the
  * FP64 matrix cores, the others from HBM/L2; 0 forces the global path.
- * Applies to later submissions and pieces on this context.  No counterpart
- * in the reference: a tuning knob. */
+ * Applies to later submissions and pieces on this context, which from then on
+ * keep to workgroups of four waves and this arena: the choice of wider ones
+ * for large systems and pieces is the library's only while the caller makes
+ * none.  No counterpart in the reference: a tuning knob. */
 int ttals_set_arena_kb(ttals_ctx* ctx, int kb);
 
 /* Local tolerance policy of later evp submissions on this context:

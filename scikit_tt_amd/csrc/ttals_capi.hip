@@ -1181,8 +1181,13 @@ int enqueue_batch(ttals_ctx* c, hipStream_t stream, const BatchArgs& B, Placemen
   }
   const SysDesc* ddesc = (const SysDesc*)dptr(m_descs);
   const int nsmall = count - nwide;
-  // both classes: the small systems on the side stream, after the wide launch
-  // has taken its CUs; the caller's stream goes on when both are done
+  // both classes: the small systems on the side stream, the wide launch enqueued
+  // first.  The fork orders the side stream after the metadata copy alone: the
+  // wide workgroups, a CU each, are likely to be placed first, not sure to be.
+  // The caller's stream goes on when both are done.  A context's side stream
+  // costs nothing where it idles, and where four contexts share the device (100
+  // to 1500 mixed requests a second) the median latency is the same as with one
+  // stream after the other, or up to 15 % lower.
   const bool both = nwide > 0 && nsmall > 0;
   if (both) HIPCHK(c, hipEventRecord(c->fork, stream));
   if (nwide > 0) {

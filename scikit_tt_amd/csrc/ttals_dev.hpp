@@ -1734,7 +1734,7 @@ __device__ void hh_block_t(const double* tau, const double* G, int kb, double* T
 // exchanges and across the waves in Yb (NB x 64 doubles), in a fixed order.
 // HH_U: 2 where the kernel must stay within 256 registers for two workgroups
 // per CU (k_als), 4 in a translation unit that defines TTALS_HH_ROWS for a
-// one-workgroup-per-CU kernel .
+// one-workgroup-per-CU kernel.
 #ifndef TTALS_HH_ROWS
 #define TTALS_HH_ROWS 2
 #endif

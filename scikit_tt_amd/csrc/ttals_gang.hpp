@@ -522,7 +522,7 @@ __device__ __forceinline__ void gang_stage1(int a, int P, int n, int b, int s, c
 // LDS.  v is read whole (it is complete in global memory), each element once;
 // the contractions after that see no global latency.  The global form
 // (gang_matvec) writes and reads both intermediates through L2 and pays a
-// round trip per K-step of each GEMM: 37.7 ms against 18.9 ms for two sweeps
+// round trip per K-step of each GEMM: 33.7 ms against 18.9 ms for two sweeps
 // of a system of order 4, n = 32, ranks 32, on 32 members (412 iterations).
 // be != 0: y = M (v + be w) for the w of the call before, whose T1 is still
 // there (stage 1 is linear), so a CG direction needs neither a barrier nor a
