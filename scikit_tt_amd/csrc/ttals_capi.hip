@@ -2265,16 +2265,17 @@ int ttals_core_product(void* stream, int r1, int m, int n, int r2, int s1, int p
   // The column form's threads each work through a chain of q's and j's (about
   // 24 ns a term, over the rows and j's of a share; a j outside the groups of
   // four counts twice), which only enough columns hide; the element form costs
-  // about half a ps per term of the whole product and 50 ns per q.  The cheaper
-  // of the two by that estimate: over 560 shapes, ranks up to 300, within 1 %
-  // of the better form on average.  A (128, 16, 16, 128) operator core times a
-  // (1, 16, 1, 1) core: 210 us by columns, 6.9 us by elements; (1, 1, 64, 200)
-  // times (1, 64, 1, 200), an inner product's first core: 364 and 9.6 us; a
-  // 1000 x 1000 matrix times a vector: 67 and 131 us (and the header of
-  // k_core_product).  Launches past the grid's limits by elements too.
+  // about half a ps per term of the whole product and 100 ns per q (50 warm, 200
+  // cold).  The cheaper of the two by that estimate: over 560 shapes, ranks up
+  // to 300, within 1.4 % of the better form on average.  A (128, 16, 16, 128)
+  // operator core times a (1, 16, 1, 1) core: 210 us by columns, 6.9 us by
+  // elements; (1, 1, 64, 200) times (1, 64, 1, 200), an inner product's first
+  // core: 364 and 9.6 us; a 1000 x 1000 matrix times a vector: 67 and 131 us
+  // (and the header of k_core_product).  Launches past the grid's limits by
+  // elements too.
   const long total = rows * s1 * p * ((long)r2 * s2);
   const double chain = (double)((rows + by - 1) / by) * n * (4 * (r2 / 4) + 2 * (r2 % 4));
-  if (chain * 48e3 > std::max((n + 2.0) * (double)total, 1e5 * n) || bx >= (1L << 24) || rows > 0x7fffffffL) {
+  if (chain * 48e3 > std::max((n + 2.0) * (double)total, 2e5 * n) || bx >= (1L << 24) || rows > 0x7fffffffL) {
     const unsigned blocks = (unsigned)std::min<long>((total + 255) / 256, 65536);
     hipLaunchKernelGGL(total < (1L << 31) ? k_core_product_elem<unsigned> : k_core_product_elem<unsigned long>,
                        dim3(blocks), dim3(256), 0, (hipStream_t)stream, r1, m, n, r2, s1, p, s2, A, X, out);
